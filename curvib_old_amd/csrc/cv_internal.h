@@ -200,10 +200,6 @@ __device__ inline int cv_wrap(int i, int m, int per) {
   return per ? (i == m - 1 ? 1 : (i == 0 ? m - 2 : i)) : i;
 }
 
-// line-solve launches of at most this many blocks (one per CU of the
-// MI355X's 256) load x with the residual (yline_reg_tile's PX)
-#define CV_PX_BLOCKS 256
-
 // XCD-aware tile order.  Work-groups are handed to the 8 XCDs of the chip
 // round-robin by linear id; this maps the blocks one XCD receives onto a
 // contiguous run of tiles (x fastest), so tiles that share halo lines share
@@ -226,6 +222,13 @@ __device__ inline void cv_xcd_runs(int R, int &tx, int &ty, int &tz) {
   tx = (int)(t % gx);
   ty = (int)((t / gx) % gy);
   tz = (int)(t / (gx * gy));
+}
+// the same for a one-dimensional grid: no division by a run-time extent
+__device__ inline int cv_xcd_line() {
+  const unsigned nb = gridDim.x, b = blockIdx.x;
+  const unsigned q = nb / CV_NXCD, rem = nb % CV_NXCD;
+  const unsigned x = b % CV_NXCD, l = b / CV_NXCD;
+  return (int)((x < rem ? x * (q + 1) : rem * (q + 1) + (x - rem) * q) + l);
 }
 __device__ inline void cv_xcd_tile(int &tx, int &ty, int &tz) {
   const unsigned gx = gridDim.x, gy = gridDim.y;

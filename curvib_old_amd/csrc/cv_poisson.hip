@@ -637,6 +637,24 @@ __global__ void __launch_bounds__(64 * YL_NC) k_yline_solve(int mx, int my, int 
   }
 }
 
+// p[i] by a 32-bit byte offset from a wavefront-uniform pointer (one address
+// register a lane for all rows); i below 2^32 / sizeof(T).  The empty asm
+// keeps the pointer in scalar registers: without it the compiler folds it
+// into one 64-bit vector address per row
+#define CV_GLOBAL __attribute__((address_space(1)))
+template <class T>
+__device__ __forceinline__ T ld32(const T *p, unsigned i) {
+  const CV_GLOBAL char *g = (const CV_GLOBAL char *)p;
+  asm("" : "+s"(g));
+  return *(const CV_GLOBAL T *)(g + (unsigned)(i * sizeof(T)));
+}
+template <class T>
+__device__ __forceinline__ void st32(T *p, unsigned i, T v) {
+  CV_GLOBAL char *g = (CV_GLOBAL char *)p;
+  asm("" : "+s"(g));
+  *(CV_GLOBAL T *)(g + (unsigned)(i * sizeof(T))) = v;
+}
+
 // register-resident line solve: block 64 lanes (i) x NC chunks along j,
 // each thread keeps the CS rows of its chunk in registers, so r, the line
 // factors and x are each read once and x written once.  Forward recurrence
@@ -644,100 +662,145 @@ __global__ void __launch_bounds__(64 * YL_NC) k_yline_solve(int mx, int my, int 
 // e_j = y_j - cp_j e_{j+1}; chunk carries resolved through LDS.
 // lines lg*64 .. lg*64+63 of the register-resident line solve, counted
 // i fastest over the (i, k) pairs of the level (a group may span two k
-// planes, so no lane idles where mx is not a multiple of 64); the chunks
-// beyond the line (blockDim.y larger than the line needs) are identity
-// maps, so the result does not depend on blockDim.y
+// planes, so no lane idles where mx is not a multiple of 64); the rows and
+// chunks beyond the line (blockDim.y larger than the line needs) are
+// identity maps, so the result does not depend on blockDim.y
+// Bound by memory: 18 (FP16 factors) to 48 bytes a row.  All loads of a chunk
+// are issued before the first is used, none behind a branch, and x while the
+// carries are exchanged: with a row's loads inside its own bounds test each
+// row waited for its own memory round trip, 16 in turn.  Per launch, before
+// and after: 12.1 M points in FP64 161 and 107 us (3.6 and 5.4 TB/s), 34.2 M
+// points with FP16 factors 145 and 127 us (4.3 and 4.9 TB/s); coarse levels of
+// up to 14 blocks 12-13 and 8-9 us
 // HL: the factors from the FP16 packs yh and yc (a 4-byte and a 2-byte
 // load per row, cp kept in registers for the backward pass); the solution
 // then carries 2^e and the caller passes omega * 2^-e
-// PX: x is loaded with r at the start (each thread reads and writes only
-// its own rows, so xi may be xo), which takes one dependent memory round
-// trip off a launch of few blocks at the cost of CS registers (launches of
-// more blocks than CUs keep PX off)
-template <class T, int CS, bool HL = false, bool PX = false>
+template <class T, int CS, bool HL = false>
 __device__ __forceinline__ void yline_reg_tile(int mx, int my, int mz, const T *r, const T *__restrict__ ya,
                                       const T *__restrict__ ip, const T *__restrict__ cp, const T *xi, T *xo,
                                       T omega, int zero_guess, int lg, const uint32_t *__restrict__ yh = nullptr,
                                       const uint16_t *__restrict__ yc = nullptr) {
   __shared__ T SA[16][64], SB[16][64];
-  const int ti = threadIdx.x, tc = threadIdx.y, nc = blockDim.y;
-  const long q0 = (long)lg * 64 + ti;
-  const bool act = q0 < (long)mx * mz;
-  const int i = act ? (int)(q0 % mx) : 0, k = act ? (int)(q0 / mx) : 0;
-  const long sj = mx;
-  const long base = (long)i + (long)mx * my * k;
+  constexpr int LB = sizeof(T) == 8 ? 8 : 16 < CS ? 16 : CS;   // rows whose loads are issued together
+  const int ti = threadIdx.x, nc = blockDim.y;
+  const int tc = __builtin_amdgcn_readfirstlane((int)threadIdx.y);   // one chunk per wavefront
+  // 32-bit throughout: the index arithmetic is a good part of a short launch
+  const unsigned q0 = (unsigned)lg * 64u + (unsigned)ti;
+  const bool act = q0 < (unsigned)mx * (unsigned)mz;
+  const unsigned k = act ? q0 / (unsigned)mx : 0u, i = act ? q0 - k * (unsigned)mx : 0u;
+  // the line's first storage index; a context needs over 256 bytes a point,
+  // so storage stays below 2^29 points on this card and 32-bit byte offsets
+  // of the lanes from a wavefront-uniform row pointer suffice
+  const unsigned base = i + (unsigned)(mx * my) * k;
   const int j0 = 1 + tc * CS;
-  const int nrow = act ? max(0, min(CS, my - 1 - j0)) : 0;
-  T av[CS], yv[CS], cv[HL ? CS : 1], xv[PX ? CS : 1];
-  if constexpr (PX) {
-#pragma unroll
-    for (int q = 0; q < CS; q++)
-      xv[q] = q < nrow && !zero_guess ? xi[base + sj * (j0 + q)] : (T)0;
-  }
+  const int nrow = max(0, min(CS, my - 1 - j0));
+  // offset of row q of the chunk; rows past the line read row my-1 and are
+  // replaced by the identity, so no load waits behind a branch
+  auto row = [&](int q) -> long { return (long)mx * min(j0 + q, my - 1); };
+  const long top = (long)mx * (my - 1);
+  T av[CS], yv[CS], xv[CS];
   // forward composite of the chunk
   T Aa = 1, Bb = 0;
+  T cv[HL ? CS : 1];
 #pragma unroll
-  for (int q = 0; q < CS; q++) {
-    if (q < nrow) {
-      const long t = base + sj * (j0 + q);
+  for (int h = 0; h < CS; h += LB) {
+    T rr[LB], pp[LB];
+    uint32_t ww[HL ? LB : 1];
+    uint16_t cc[HL ? LB : 1];
+#pragma unroll
+    for (int q = 0; q < LB; q++) {
+      const long o = row(h + q);
+      rr[q] = ld32(r + o, base);
       if constexpr (HL) {
-        const uint32_t w = yh[t];
-        av[q] = half_lo(w);
-        yv[q] = r[t] * half_hi(w);
-        cv[q] = half_lo((uint32_t)yc[t]);
+        ww[q] = ld32(yh + o, base);
+        cc[q] = ld32(yc + o, base);
       } else {
-        av[q] = ya[t];
-        yv[q] = r[t] * ip[t];
+        av[h + q] = ld32(ya + o, base);
+        pp[q] = ld32(ip + o, base);
       }
-      Aa = av[q] * Aa;
-      Bb = av[q] * Bb + yv[q];
+    }
+#pragma unroll
+    for (int q = 0; q < LB; q++) {
+      const bool in = h + q < nrow;
+      if constexpr (HL) {
+        av[h + q] = half_lo(ww[q]);
+        pp[q] = half_hi(ww[q]);
+        cv[h + q] = half_lo((uint32_t)cc[q]);
+      }
+      av[h + q] = in ? av[h + q] : (T)1;
+      yv[h + q] = in ? rr[q] * pp[q] : (T)0;
+      Aa = av[h + q] * Aa;
+      Bb = av[h + q] * Bb + yv[h + q];
     }
   }
   SA[tc][ti] = Aa; SB[tc][ti] = Bb;
   __syncthreads();
   T y = 0;
-  for (int q = 0; q < tc; q++) y = SA[q][ti] * y + SB[q][ti];
+#pragma unroll
+  for (int q = 0; q < 15; q++) {
+    const T a = SA[q][ti], b = SB[q][ti];
+    y = q < tc ? a * y + b : y;
+  }
+#pragma unroll
+  for (int q = 0; q < CS; q++) {
+    y = yv[q] + av[q] * y;
+    yv[q] = y;
+  }
+  // the backward multipliers and x, in flight while the block meets
+  T xe = 0;
 #pragma unroll
   for (int q = 0; q < CS; q++)
-    if (q < nrow) { y = yv[q] + av[q] * y; yv[q] = y; }
+    if constexpr (!HL) av[q] = ld32(cp + row(q), base);
+#pragma unroll
+  for (int q = 0; q < CS; q++) xv[q] = 0;
+  T xt = 0;
+  constexpr bool XE = CS * sizeof(T) <= 32;   // registers allow x beside the factors
+  auto load_x = [&]() {
+#pragma unroll
+    for (int q = 0; q < CS; q++) xv[q] = ld32(xi + row(q), base);
+    if (tc == 0) xe = ld32(xi, base);
+    if (tc == nc - 1) xt = ld32(xi + top, base);
+  };
+  if (XE && !zero_guess) load_x();
   __syncthreads();
   // backward composite, from the chunk's top row down
   Aa = 1; Bb = 0;
 #pragma unroll
   for (int q = CS - 1; q >= 0; q--) {
-    if (q < nrow) {
-      if constexpr (HL) av[q] = -cv[q];
-      else av[q] = -cp[base + sj * (j0 + q)];
-      Aa = av[q] * Aa;
-      Bb = av[q] * Bb + yv[q];
-    }
+    const bool in = q < nrow;
+    if constexpr (HL) av[q] = in ? -cv[q] : (T)1;
+    else av[q] = in ? -av[q] : (T)1;
+    yv[q] = in ? yv[q] : (T)0;
+    Aa = av[q] * Aa;
+    Bb = av[q] * Bb + yv[q];
   }
   SA[tc][ti] = Aa; SB[tc][ti] = Bb;
+  if (!XE && !zero_guess) load_x();
   __syncthreads();
   T e = 0;
-  for (int q = nc - 1; q > tc; q--) e = SA[q][ti] * e + SB[q][ti];
+#pragma unroll
+  for (int q = 15; q > 0; q--) {
+    const T a = SA[q][ti], b = SB[q][ti];
+    e = q > tc && q < nc ? a * e + b : e;
+  }
   if (!act) return;
 #pragma unroll
   for (int q = CS - 1; q >= 0; q--) {
-    if (q < nrow) {
-      const long t = base + sj * (j0 + q);
-      e = yv[q] + av[q] * e;
-      if constexpr (PX) xo[t] = xv[q] + omega * e;
-      else xo[t] = (zero_guess ? (T)0 : xi[t]) + omega * e;
-    }
+    e = yv[q] + av[q] * e;
+    if (q < nrow) st32(xo + row(q), base, xv[q] + omega * e);
   }
-  if (tc == 0) xo[base] = zero_guess ? (T)0 : xi[base];
-  if (tc == nc - 1) xo[base + sj * (my - 1)] = zero_guess ? (T)0 : xi[base + sj * (my - 1)];
+  if (tc == 0) st32(xo, base, xe);
+  if (tc == nc - 1) st32(xo + top, base, xt);
 }
 
-template <class T, int CS, bool HL = false, bool PX = false>
-__global__ void __launch_bounds__(1024) k_yline_reg(int mx, int my, int mz, const T *r, const T *__restrict__ ya,
+// waves per SIMD: two blocks of 1024 threads per CU where 16 FP32 rows fit 64
+// registers, one for the wider rows
+template <class T, int CS, bool HL = false>
+__global__ void __launch_bounds__(1024, sizeof(T) == 4 && CS <= 16 ? 8 : 4) k_yline_reg(int mx, int my, int mz, const T *r, const T *__restrict__ ya,
                                                    const T *__restrict__ ip, const T *__restrict__ cp,
                                                    const T *xi, T *xo, T omega, int zero_guess,
                                                    const uint32_t *__restrict__ yh, const uint16_t *__restrict__ yc) {
-  int lg, by, bz;
-  cv_xcd_tile(lg, by, bz);
-  yline_reg_tile<T, CS, HL, PX>(mx, my, mz, r, ya, ip, cp, xi, xo, omega, zero_guess, lg, yh, yc);
+  yline_reg_tile<T, CS, HL>(mx, my, mz, r, ya, ip, cp, xi, xo, omega, zero_guess, cv_xcd_line(), yh, yc);
 }
 
 // ------------------------------------------------------------------
@@ -1479,17 +1542,9 @@ static void line_solve(cv_ctx *c, int l, const T *r, const T *xi, T *xo, T *tmp,
     if constexpr (sizeof(T) == 4) {
       if (hl) {
         const T omh = om * A.ysc;
-        // at most one block per CU: x loaded up front
-        const bool px = g.x <= CV_PX_BLOCKS;
-        if (cs == 8 && px)
-          hipLaunchKernelGGL((k_yline_reg<T, 8, true, true>), g, b, 0, c->stream, L.d.mx, L.d.my, L.d.mz, r, A.ylo,
-                             A.yip, A.ycp, xi, xo, omh, zg ? 1 : 0, A.yh, A.yc);
-        else if (cs == 8)
+        if (cs == 8)
           hipLaunchKernelGGL((k_yline_reg<T, 8, true>), g, b, 0, c->stream, L.d.mx, L.d.my, L.d.mz, r, A.ylo, A.yip,
                              A.ycp, xi, xo, omh, zg ? 1 : 0, A.yh, A.yc);
-        else if (px)
-          hipLaunchKernelGGL((k_yline_reg<T, 16, true, true>), g, b, 0, c->stream, L.d.mx, L.d.my, L.d.mz, r, A.ylo,
-                             A.yip, A.ycp, xi, xo, omh, zg ? 1 : 0, A.yh, A.yc);
         else
           hipLaunchKernelGGL((k_yline_reg<T, 16, true>), g, b, 0, c->stream, L.d.mx, L.d.my, L.d.mz, r, A.ylo, A.yip,
                              A.ycp, xi, xo, omh, zg ? 1 : 0, A.yh, A.yc);
