@@ -75,9 +75,9 @@ __global__ void __launch_bounds__(LEG_NT) kb_leg(const BCase *__restrict__ cs, u
     __syncthreads();   // every thread has read the previous ticket
     if (tid == 0) s_tk = __hip_atomic_fetch_add(lg.ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     __syncthreads();
-    const uint32_t tk = s_tk;
+    const uint32_t tk = (uint32_t)__builtin_amdgcn_readfirstlane((int)s_tk);   // uniform: scalar descriptors below
     if ((long)tk >= lg.ntk) break;
-    const uint32_t e = lg.ord[tk];
+    const uint32_t e = (uint32_t)__builtin_amdgcn_readfirstlane((int)lg.ord[tk]);
     const int c = LEG_CASE(e), p = LEG_PHASE(e), it = LEG_ITEM(e);
     // a case outside the mask neither waits nor signals: all its items skip
     if (!((on >> c) & 1ull)) continue;
@@ -111,7 +111,7 @@ __global__ void __launch_bounds__(LEG_NT) kb_leg(const BCase *__restrict__ cs, u
     switch (P.kind) {
       case PK_STEN: {
         const int gx = (A.mx + LEG_TX - 2) / (LEG_TX - 1), gy = (A.my + LEG_TY - 1) / LEG_TY;
-        stencil_tile<T, 1, LEG_TY, HG, HG, LEG_TX>(A, x, bvec<T>(C, d, BB, 0), bvec<T>(C, d, BR, 0), A.dinv, (T)0,
+        stencil_tile<T, 1, LEG_TY, HG, LEG_TX>(A, x, bvec<T>(C, d, BB, 0), bvec<T>(C, d, BR, 0), A.dinv, (T)0,
                                                      kc, it % gx, (it / gx) % gy, it / (gx * gy));
         break;
       }

@@ -122,7 +122,7 @@ __global__ void __launch_bounds__(TW * 4) kb_stencil(BK_ARGS, int d, int sx, int
   const OpV<T> A = bop<T>(C, d);
   const int gx = C.lev[d].sgx, gy = C.lev[d].sgy, jj = ctl->jj;
   const int bx = lb % gx, by = (lb / gx) % gy, bz = lb / (gx * gy);
-  stencil_tile<T, MODE, 4, true, HG, TW, TX>(A, (const TX *)bvec<TX>(C, d, sx, jj),
+  stencil_tile<T, MODE, 4, HG, TW, TX>(A, (const TX *)bvec<TX>(C, d, sx, jj),
                                      MODE >= 1 ? bvec<T>(C, d, sb, jj) : (const T *)nullptr, bvec<T>(C, d, sy, jj),
                                      A.dinv, (T)0, C.lev[d].kc, bx, by, bz);
 }
@@ -908,7 +908,7 @@ extern "C" int cv_batch_create(cv_ctx *const *cases, int ncases, cv_batch **out)
       b.isc = L.d.isc; b.jsc = L.d.jsc; b.ksc = L.d.ksc;
       b.n = L.d.n;
       b.inv_nf = x->nfluid[l] > 0 ? 1.0 / x->nfluid[l] : 0.0;
-      b.kc = stencil_kchunk_batch(L.d.mz);
+      b.kc = stencil_fit(stencil_kchunk_batch(L.d.mz), L.d);
       b.sgx = (L.d.mx + B->tw - 2) / (B->tw - 1); b.sgy = (L.d.my + 3) / 4; b.sgz = (L.d.mz + b.kc - 1) / b.kc;
       b.lgx = (int)(((long)L.d.mx * L.d.mz + 63) / 64);
       const int rows = L.d.my - 2;

@@ -244,74 +244,110 @@ __global__ void __launch_bounds__(BS) k_jacobi(OpV<T> A, const T *__restrict__ x
 // ------------------------------------------------------------------
 
 // one face flux from its two cells (xl, xu) and the four neighbours of
-// each tangential axis: (+f, +e+f, -f, +e-f)
+// each tangential axis: (+f, +e+f, -f, +e-f).  The cross modes pick operands
+// instead of branching: a one-sided rule takes the two cells for the missing
+// pair, a dropped one leaves F
+template <class T>
+__device__ inline T tile_cross(T F, T xl, T xu, int m, T g, T a, T b, T c, T d) {
+  const bool lo = m == XM_LOWER, up = m == XM_UPPER;
+  const T s = (lo ? xl : a) + (lo ? xu : b) - (up ? xl : c) - (up ? xu : d);
+  const T f = F + g * (lo || up ? (T)0.5 : (T)0.25) * s;
+  return m == XM_DROP ? F : f;
+}
 template <class T>
 __device__ inline T tile_flux(T xl, T xu, T gdd, uint32_t w, int sh, T g0, T a0, T b0, T c0, T d0, T g1, T a1, T b1,
                               T c1, T d1) {
   T F = gdd * (xu - xl);
-  const int m0 = (w >> sh) & 3u, m1 = (w >> (sh + 2)) & 3u;
-  if (m0 == XM_CENTRAL) F += g0 * (T)0.25 * (a0 + b0 - c0 - d0);
-  else if (m0 == XM_LOWER) F += g0 * (T)0.5 * (xl + xu - c0 - d0);
-  else if (m0 == XM_UPPER) F += g0 * (T)0.5 * (a0 + b0 - xl - xu);
-  if (m1 == XM_CENTRAL) F += g1 * (T)0.25 * (a1 + b1 - c1 - d1);
-  else if (m1 == XM_LOWER) F += g1 * (T)0.5 * (xl + xu - c1 - d1);
-  else if (m1 == XM_UPPER) F += g1 * (T)0.5 * (a1 + b1 - xl - xu);
-  return F;
+  F = tile_cross<T>(F, xl, xu, (w >> sh) & 3u, g0, a0, b0, c0, d0);
+  return tile_cross<T>(F, xl, xu, (w >> (sh + 2)) & 3u, g1, a1, b1, c1, d1);
 }
 
 // k-face flux between planes P (k) and Q (k+1) at LDS column c, row r;
 // g6, g7, g8 of the face; ST_TC: the LDS row stride (tile width + 2)
 template <class T, int ST_TC>
 __device__ inline T tile_flux_k(const T *P, const T *Q, int c, int r, uint32_t w, T g6, T g7, T g8) {
-  if (!(w & (1u << 11))) return (T)0;
   const int o = r * ST_TC + c;
-  return tile_flux<T>(P[o], Q[o], g8, w, 12, g6, P[o + 1], Q[o + 1], P[o - 1], Q[o - 1],
+  const T F = tile_flux<T>(P[o], Q[o], g8, w, 12, g6, P[o + 1], Q[o + 1], P[o - 1], Q[o - 1],
                       g7, P[o + ST_TC], Q[o + ST_TC], P[o - ST_TC], Q[o - ST_TC]);
+  return (w & (1u << 11)) ? F : (T)0;
 }
 // j-face flux between rows r and r+1 of plane P (M = k-1, Q = k+1)
 template <class T, int ST_TC>
 __device__ inline T tile_flux_j(const T *M, const T *P, const T *Q, int c, int r, uint32_t w, T g3, T g4, T g5) {
-  if (!(w & (1u << 6))) return (T)0;
   const int o = r * ST_TC + c, u = o + ST_TC;
-  return tile_flux<T>(P[o], P[u], g4, w, 7, g3, P[o + 1], P[u + 1], P[o - 1], P[u - 1],
+  const T F = tile_flux<T>(P[o], P[u], g4, w, 7, g3, P[o + 1], P[u + 1], P[o - 1], P[u - 1],
                       g5, Q[o], Q[u], M[o], M[u]);
+  return (w & (1u << 6)) ? F : (T)0;
 }
 // i-face flux between columns c and c+1 of plane P
 template <class T, int ST_TC>
 __device__ inline T tile_flux_i(const T *M, const T *P, const T *Q, int c, int r, uint32_t w, T g0, T g1, T g2) {
-  if (!(w & (1u << 1))) return (T)0;
   const int o = r * ST_TC + c;
-  return tile_flux<T>(P[o], P[o + 1], g0, w, 2, g1, P[o + ST_TC], P[o + ST_TC + 1], P[o - ST_TC], P[o - ST_TC + 1],
+  const T F = tile_flux<T>(P[o], P[o + 1], g0, w, 2, g1, P[o + ST_TC], P[o + ST_TC + 1], P[o - ST_TC], P[o - ST_TC + 1],
                       g2, Q[o], Q[o + 1], M[o], M[o + 1]);
+  return (w & (1u << 1)) ? F : (T)0;
 }
 
 // FP16 halves of packed coefficient words, widened to FP32 (exact)
 __device__ inline float half_lo(uint32_t w) { return (float)__builtin_bit_cast(_Float16, (unsigned short)(w & 0xffffu)); }
 __device__ inline float half_hi(uint32_t w) { return (float)__builtin_bit_cast(_Float16, (unsigned short)(w >> 16)); }
 
-// operator word and face coefficients of one cell, loaded a plane ahead;
-// in FP32 (where registers allow it) also aj, b and dinv
+// Bounds-checked loads and stores through a buffer descriptor: a lane whose
+// offset lies past the end (CV_OOB) reads 0 or stores nothing, without a
+// branch and without touching memory.  Branches around loads cost far more
+// than the loads: after them the compiler no longer knows how many loads are
+// in flight and waits for all, the next plane's prefetch included.
+typedef __amdgpu_buffer_rsrc_t CvBuf;
+#define CV_OOB 0xfffffff0u
+__device__ __forceinline__ CvBuf cv_buf(const void *p, unsigned long bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), 0, (int)(bytes < CV_OOB ? bytes : CV_OOB), 0x00020000);
+}
+typedef uint32_t cv_u2 __attribute__((ext_vector_type(2)));
+typedef uint32_t cv_u4 __attribute__((ext_vector_type(4)));
 template <class T>
+__device__ __forceinline__ T cv_bld(CvBuf b, unsigned off, unsigned so) {
+  static_assert(sizeof(T) == 4 || sizeof(T) == 8 || sizeof(T) == 16, "4, 8 or 16 bytes");
+  if constexpr (sizeof(T) == 4) return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b32(b, off, so, 0));
+  else if constexpr (sizeof(T) == 8) return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b64(b, off, so, 0));
+  else return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b128(b, off, so, 0));
+}
+template <class T>
+__device__ __forceinline__ void cv_bst(CvBuf b, T v, unsigned off, unsigned so) {
+  if constexpr (sizeof(T) == 4) __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), b, off, so, 0);
+  else __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(cv_u2, v), b, off, so, 0);
+}
+
+// one cell's operands as loaded a plane ahead: the operator word, the face
+// coefficients (HG: the FP16 packs, decoded only when the plane is computed),
+// aj, b, dinv; the operator word and j-face coefficients of the cell below
+// the tile (row 0); the cell's own x where the tile holds the periodic image
+template <class T, bool HG>
 struct StCell {
-  uint32_t w, wb;        // operator words of the cell and (row 0) of the cell below the tile
+  uint32_t w, wb;
   T g[9], gb[3];
-  T aj, b, dv;
-  // FP16 packs as loaded (HG): decoded into w, g, aj, wb, gb only when the
-  // plane is computed, so the prefetch a plane ahead stays in flight
-  uint4 ha;
-  uint2 hb, hbb;
+  T aj, b, dv, xg;
+};
+template <class T>
+struct StCell<T, true> {
+  cv_u4 ha;
+  cv_u2 hb, hbb;
+  T b, dv, xg;
 };
 
-// TY: rows per block (block TW x TY); PFB: prefetch the row-0 face below
-// the tile with the cells (keeps the row-0 wave off the barrier's critical
-// path at the cost of registers); HG: face coefficients from the FP16
+// TY: rows per block (block TW x TY); HG: face coefficients from the FP16
 // packs instead of g, aj; TW: lanes per tile row, 64 (one wavefront per
 // row) or 32 (two rows per wavefront; the i-face shuffle stays within a
 // row); remap: XCD-aware tile order
 // one tile (bx, by, bz) of the stencil: (TW-1) x TY cells of kchunk planes
 // TX: element type of x (FP32 preconditioned vectors under the FP64 apply
 // of the mixed solve; widened exactly on load)
-template <class T, int MODE, int TY, bool PFB, bool HG = false, int TW = 64, class TX = T>
+// Bound by memory: 36 (FP16 packs) to 108 (FP64) bytes a point; 78 registers
+// with the packs (6 waves per SIMD), 159 in FP64 (3).  Residual per launch
+// with branches around the loads and now: FP16 packs on 34.2 M points 262 and
+// 253 us (4.9 TB/s), on 9.7 M 86 and 74 us, on 1.3 M 21 and 16 us; FP64 on
+// 12.1 M 296 and 285 us.  Capping the registers for 7 waves (FP16) or 4
+// (FP64) spills: 309 us, and 1282 us for an apply that takes 687
+template <class T, int MODE, int TY, bool HG = false, int TW = 64, class TX = T>
 __device__ __forceinline__ void stencil_tile(const OpV<T> &A, const TX *__restrict__ x, const T *__restrict__ b,
                                     T *__restrict__ y, const T *__restrict__ dinv, T omega, int kchunk, int bx,
                                     int by, int bz, int color = -1) {
@@ -319,7 +355,7 @@ __device__ __forceinline__ void stencil_tile(const OpV<T> &A, const TX *__restri
   constexpr int ST_TC = TW + 2;
   constexpr int TR = TY + 2, NT = TR * ST_TC, NTH = TW * TY;
   static_assert(2 * NTH >= NT, "two tile entries per thread must cover a plane");
-  __shared__ T X[4][NT];
+  __shared__ T X[4][2 * NTH];
   __shared__ T FJ[2][TY][TW];
   const int L = threadIdx.x, R = threadIdx.y;
   const int tid = R * TW + L;
@@ -327,209 +363,190 @@ __device__ __forceinline__ void stencil_tile(const OpV<T> &A, const TX *__restri
   const int i0 = (TW - 1) * bx, j0 = TY * by;
   const int k0 = kchunk * bz, k1 = min(k0 + kchunk, mz);
   const int gi = i0 - 1 + L, gj = j0 + R;
-  const bool in_i = gi >= 0 && gi < mx, in_j = gj < my;
-  const bool cell = in_i && in_j;
+  const bool cell = gi >= 0 && gi < mx && gj < my;
   const bool out = L >= 1 && cell;
   const bool row0 = out && R == 0 && gj >= 1;
-  const long pl = (long)mx * my;
+  const unsigned pl = (unsigned)mx * (unsigned)my;
+  const unsigned long n = (unsigned long)pl * (unsigned)mz;
   const int c = L + 1, r = R + 1;
-  const long tij = (long)gi + (long)mx * gj;
+  const unsigned tij = (unsigned)gi + (unsigned)mx * (unsigned)gj;
 
-  // this thread's share of a tile plane: entries tid and e1 = tid + NTH
-  const int e1 = tid + NTH;
-  long off0 = 0, off1 = 0;
-  bool ok0, ok1;
-  {
-    int rr = tid / ST_TC, cc = tid - rr * ST_TC;
-    int ii = i0 - 2 + cc, jj = j0 - 1 + rr;
-    ok0 = tid < NT && ii >= 0 && ii < mx && jj >= 0 && jj < my;
-    if (ok0) off0 = (long)mx * jj + cv_wrap(ii, mx, A.xper);
-    rr = e1 / ST_TC; cc = e1 - rr * ST_TC;
-    ii = i0 - 2 + cc; jj = j0 - 1 + rr;
-    ok1 = e1 < NT && ii >= 0 && ii < mx && jj >= 0 && jj < my;
-    if (ok1) off1 = (long)mx * jj + cv_wrap(ii, mx, A.xper);
+  // x over the whole storage; the other arrays from plane kb on, so that
+  // their byte offsets stay within 32 bits for every grid (stencil_fit)
+  const int kb = max(k0 - 1, 0);
+  const unsigned long nb_ = n - (unsigned long)pl * (unsigned)kb;
+  const CvBuf Bx = cv_buf(x, n * sizeof(TX));
+  auto plane_buf = [&](const void *p, unsigned sz) {
+    return cv_buf((const char *)p + (unsigned long)pl * (unsigned)kb * sz, nb_ * sz);
+  };
+  // offsets in elements, CV_OOB / 16 and beyond never valid
+  auto boff = [](bool ok, unsigned t, unsigned sz) { return ok ? t * sz : CV_OOB; };
+
+  // this thread's share of a tile plane: entries tid and tid + NTH
+  unsigned off[2];
+#pragma unroll
+  for (int q = 0; q < 2; q++) {
+    const int e = tid + q * NTH;
+    const int rr = e / ST_TC, cc = e - rr * ST_TC;
+    const int ii = i0 - 2 + cc, jj = j0 - 1 + rr;
+    const bool ok = e < NT && ii >= 0 && ii < mx && jj >= 0 && jj < my;
+    off[q] = boff(ok, (unsigned)mx * (unsigned)jj + (unsigned)cv_wrap(ii, mx, A.xper), sizeof(TX));
   }
   // x values travel in their own type until they are stored to LDS, so a
   // narrower x (FP32 under the FP64 apply) is widened only when its
-  // prefetch is consumed, not when it is issued
-  auto fetch_x = [&](int gk, TX &v0, TX &v1) {
-    const bool kin = gk >= 0 && gk < mz;
-    const long kb = kin ? pl * cv_wrap(gk, mz, A.zper) : 0;
-    v0 = (kin && ok0) ? x[kb + off0] : (TX)0;
-    v1 = (kin && ok1) ? x[kb + off1] : (TX)0;
+  // prefetch is consumed, not when it is issued.  Planes past kmax are not
+  // loaded (0)
+  auto fetch_x = [&](int gk, int kmax, TX (&v)[2]) {
+    const bool kin = gk >= 0 && gk < mz && gk <= kmax;
+    const unsigned so = kin ? pl * (unsigned)cv_wrap(gk, mz, A.zper) * (unsigned)sizeof(TX) : 0u;
+    const unsigned inv = kin ? 0u : CV_OOB;
+#pragma unroll
+    for (int q = 0; q < 2; q++) v[q] = cv_bld<TX>(Bx, off[q] | inv, so);
   };
-  auto store_x = [&](int gk, TX v0, TX v1) {
+  auto store_x = [&](int gk, const TX (&v)[2]) {
     T *S = X[(gk + 4) & 3];
-    if (tid < NT) S[tid] = (T)v0;
-    if (e1 < NT) S[e1] = (T)v1;
+    S[tid] = (T)v[0];
+    S[tid + NTH] = (T)v[1];
   };
-  constexpr bool PF = sizeof(T) == 4;      // prefetch aj, b, dinv with the cell
-  auto gco = [&](int q, long t) -> T {
+  const unsigned oc = boff(cell, tij, 1), oo = boff(out, tij, 1), ob = boff(row0, tij - (unsigned)mx, 1);
+  auto sc = [](unsigned o, unsigned sz) { return o == CV_OOB ? CV_OOB : o * sz; };
+  const unsigned oT = sc(oo, sizeof(T)), cT = sc(oc, sizeof(T)), bT = sc(ob, sizeof(T));
+  // lanes whose tile entry is a periodic image of another cell
+  const bool ghost_i = A.xper && (gi == 0 || gi == mx - 1);
+  const unsigned gxo = out ? tij * (unsigned)sizeof(TX) : CV_OOB;
+  auto fetch_cell = [&](int gk, StCell<T, HG> &C) {
+    const unsigned kq = (unsigned)(gk - kb) * pl;
+    const bool kin = gk < k1;
+    const unsigned inv = kin ? 0u : CV_OOB;
+    const unsigned sk = kin ? kq : 0u;
     if constexpr (HG) {
-      if (q >= 3 && q <= 5) {
-        const uint2 hb = A.hB[t];
-        return q == 3 ? half_lo(hb.x) : q == 4 ? half_hi(hb.x) : half_lo(hb.y);
-      }
-      const uint4 ha = A.hA[t];
-      return q == 0 ? half_lo(ha.x) : q == 1 ? half_hi(ha.x) : q == 2 ? half_lo(ha.y)
-           : q == 6 ? half_hi(ha.y) : q == 7 ? half_lo(ha.z) : half_hi(ha.z);
+      C.ha = cv_bld<cv_u4>(plane_buf(A.hA, 16), sc(oc, 16) | inv, sk * 16u);
+      C.hb = cv_bld<cv_u2>(plane_buf(A.hB, 8), sc(oc, 8) | inv, sk * 8u);
+      C.hbb = cv_bld<cv_u2>(plane_buf(A.hB, 8), sc(ob, 8) | inv, sk * 8u);
     } else {
-      return A.g[q][t];
-    }
-  };
-  auto ajo = [&](long t) -> T {
-    if constexpr (HG) return __uint_as_float(A.hA[t].w);
-    else return A.aj[t];
-  };
-  auto wo = [&](long t) -> uint32_t {
-    if constexpr (HG) return A.hB[t].y >> 16;
-    else return A.fl[t];
-  };
-  auto fetch_cell = [&](int gk, StCell<T> &C) {
-    C.w = 0u;
+      C.w = cv_bld<uint32_t>(plane_buf(A.fl, 4), sc(oc, 4) | inv, sk * 4u);
 #pragma unroll
-    for (int q = 0; q < 9; q++) C.g[q] = (T)0;
-    C.aj = C.b = C.dv = (T)0;
-    C.wb = 0u;
-    C.gb[0] = C.gb[1] = C.gb[2] = (T)0;
-    if constexpr (HG) {
-      C.ha = make_uint4(0u, 0u, 0u, 0u);
-      C.hb = C.hbb = make_uint2(0u, 0u);
-    }
-    if (!cell) return;
-    const long t = tij + pl * gk;
-    if constexpr (HG) {
-      C.ha = A.hA[t];
-      C.hb = A.hB[t];
-    } else {
-      C.w = A.fl[t];
+      for (int q = 0; q < 9; q++) C.g[q] = cv_bld<T>(plane_buf(A.g[q], sizeof(T)), cT | inv, sk * (unsigned)sizeof(T));
+      C.wb = cv_bld<uint32_t>(plane_buf(A.fl, 4), sc(ob, 4) | inv, sk * 4u);
 #pragma unroll
-      for (int q = 0; q < 9; q++) C.g[q] = A.g[q][t];
+      for (int q = 0; q < 3; q++)
+        C.gb[q] = cv_bld<T>(plane_buf(A.g[3 + q], sizeof(T)), bT | inv, sk * (unsigned)sizeof(T));
+      C.aj = cv_bld<T>(plane_buf(A.aj, sizeof(T)), oT | inv, sk * (unsigned)sizeof(T));
     }
-    if (PF && out) {
-      if constexpr (!HG) C.aj = A.aj[t];
-      if (MODE >= 1) C.b = b[t];
-      if (MODE == 2) C.dv = dinv[t];
-    }
-    if (PFB && row0) {
-      if constexpr (HG) {
-        C.hbb = A.hB[t - mx];
-      } else {
-        C.wb = A.fl[t - mx];
-        C.gb[0] = A.g[3][t - mx]; C.gb[1] = A.g[4][t - mx]; C.gb[2] = A.g[5][t - mx];
-      }
-    }
+    if (MODE >= 1) C.b = cv_bld<T>(plane_buf(b, sizeof(T)), oT | inv, sk * (unsigned)sizeof(T));
+    if (MODE == 2) C.dv = cv_bld<T>(plane_buf(dinv, sizeof(T)), oT | inv, sk * (unsigned)sizeof(T));
+    const bool gh = kin && (ghost_i || (A.zper && (gk == 0 || gk == mz - 1)));
+    C.xg = (T)cv_bld<TX>(Bx, gh ? gxo : CV_OOB, kin ? pl * (unsigned)gk * (unsigned)sizeof(TX) : 0u);
   };
 
-  // the FP16 packs of a fetched cell into its operands (zero where the cell
-  // lies outside the grid: the packs were cleared then)
-  auto decode_cell = [&](StCell<T> &C) {
-    if constexpr (HG) {
-      const uint4 ha = C.ha;
-      const uint2 hb = C.hb, hbb = C.hbb;
-      C.w = hb.y >> 16;
-      C.g[0] = half_lo(ha.x); C.g[1] = half_hi(ha.x); C.g[2] = half_lo(ha.y);
-      C.g[3] = half_lo(hb.x); C.g[4] = half_hi(hb.x); C.g[5] = half_lo(hb.y);
-      C.g[6] = half_hi(ha.y); C.g[7] = half_lo(ha.z); C.g[8] = half_hi(ha.z);
-      C.aj = out ? __uint_as_float(ha.w) : (T)0;
-      if (PFB && row0) {
-        C.wb = hbb.y >> 16;
-        C.gb[0] = half_lo(hbb.x); C.gb[1] = half_hi(hbb.x); C.gb[2] = half_lo(hbb.y);
-      }
-    }
-  };
-
-  // prologue: planes k0-1 .. k0+1 in LDS, plane k0+2 and the cells of k0 in
-  // registers.  The chunk reads planes k0-1 .. k1 only (plane gk+1 is the
-  // last neighbour of plane gk), so planes past k1 are neither loaded nor
-  // stored: the next chunk loads them itself
-  TX xa, xb;
-  fetch_x(k0 - 1, xa, xb); store_x(k0 - 1, xa, xb);
-  fetch_x(k0, xa, xb); store_x(k0, xa, xb);
-  fetch_x(k0 + 1, xa, xb); store_x(k0 + 1, xa, xb);
-  TX xn0 = (TX)0, xn1 = (TX)0;
-  if (k0 + 2 <= k1) fetch_x(k0 + 2, xn0, xn1);
-  StCell<T> cur;
+  // prologue: planes k0-1 .. k0+2, the cells of k0 and the k-face
+  // coefficients of the plane below, all in flight together.  The chunk
+  // reads planes k0-1 .. k1 only (plane gk+1 is the last neighbour of plane
+  // gk); the next chunk loads those past k1 itself
+  TX xp[3][2], xn[2];
+#pragma unroll
+  for (int q = 0; q < 3; q++) fetch_x(k0 - 1 + q, mz, xp[q]);
+  StCell<T, HG> cur;
   fetch_cell(k0, cur);
-  __syncthreads();
   T fk_lo = (T)0;
-  if (out && k0 >= 1) {
-    const long t = tij + pl * (k0 - 1);
-    fk_lo = tile_flux_k<T, ST_TC>(X[(k0 - 1 + 4) & 3], X[(k0 + 4) & 3], c, r, wo(t), gco(6, t), gco(7, t), gco(8, t));
+  uint32_t wl;
+  T gl[3];
+  {
+    const unsigned inv = k0 >= 1 ? 0u : CV_OOB;   // kb = k0 - 1
+    if constexpr (HG) {
+      const cv_u4 ha = cv_bld<cv_u4>(plane_buf(A.hA, 16), sc(oo, 16) | inv, 0u);
+      const cv_u2 hb = cv_bld<cv_u2>(plane_buf(A.hB, 8), sc(oo, 8) | inv, 0u);
+      wl = hb.y >> 16;
+      gl[0] = half_hi(ha.y); gl[1] = half_lo(ha.z); gl[2] = half_hi(ha.z);
+    } else {
+      wl = cv_bld<uint32_t>(plane_buf(A.fl, 4), sc(oo, 4) | inv, 0u);
+#pragma unroll
+      for (int q = 0; q < 3; q++) gl[q] = cv_bld<T>(plane_buf(A.g[6 + q], sizeof(T)), oT | inv, 0u);
+    }
   }
-  for (int gk = k0; gk < k1; gk++) {
-    TX xq0 = (TX)0, xq1 = (TX)0;
-    if (gk + 3 <= k1) fetch_x(gk + 3, xq0, xq1);
-    StCell<T> nxt;
-    if (gk + 1 < k1) fetch_cell(gk + 1, nxt);
-    const long t = tij + pl * gk;
+  fetch_x(k0 + 2, k1, xn);
+#pragma unroll
+  for (int q = 0; q < 3; q++) store_x(k0 - 1 + q, xp[q]);
+  __syncthreads();
+  fk_lo = tile_flux_k<T, ST_TC>(X[(k0 - 1 + 4) & 3], X[(k0 + 4) & 3], c, r, wl, gl[0], gl[1], gl[2]);
+  const CvBuf By = plane_buf(y, sizeof(T));
+  // one plane: cur and xn hold this plane's cells and x plane gk+2, nxt and xq
+  // take the next ones.  The two register sets swap roles from plane to plane
+  // (the loop below); moving one into the other would wait for its loads
+  auto plane = [&](int gk, const StCell<T, HG> &cur, StCell<T, HG> &nxt, const TX (&xn)[2], TX (&xq)[2]) {
+    fetch_x(gk + 3, k1, xq);
+    fetch_cell(gk + 1, nxt);
     const T *Pm = X[(gk - 1 + 4) & 3], *P = X[(gk + 4) & 3], *Q = X[(gk + 1 + 4) & 3];
-    decode_cell(cur);
-    const uint32_t w = cur.w;
-    const T fi = cell ? tile_flux_i<T, ST_TC>(Pm, P, Q, c, r, w, cur.g[0], cur.g[1], cur.g[2]) : (T)0;
-    T fj = (T)0, fk = (T)0, fj_lo = (T)0;
-    if (out) {
-      fj = tile_flux_j<T, ST_TC>(Pm, P, Q, c, r, w, cur.g[3], cur.g[4], cur.g[5]);
-      fk = tile_flux_k<T, ST_TC>(P, Q, c, r, w, cur.g[6], cur.g[7], cur.g[8]);
-      if (row0) {
-        if (PFB) {
-          fj_lo = tile_flux_j<T, ST_TC>(Pm, P, Q, c, r - 1, cur.wb, cur.gb[0], cur.gb[1], cur.gb[2]);
-        } else {
-          const long tb = t - mx;
-          fj_lo = tile_flux_j<T, ST_TC>(Pm, P, Q, c, r - 1, wo(tb), gco(3, tb), gco(4, tb), gco(5, tb));
-        }
-      }
+    uint32_t w, wb;
+    T g[9], gb[3], ajc;
+    if constexpr (HG) {
+      const cv_u4 ha = cur.ha;
+      const cv_u2 hb = cur.hb, hbb = cur.hbb;
+      w = hb.y >> 16;
+      g[0] = half_lo(ha.x); g[1] = half_hi(ha.x); g[2] = half_lo(ha.y);
+      g[3] = half_lo(hb.x); g[4] = half_hi(hb.x); g[5] = half_lo(hb.y);
+      g[6] = half_hi(ha.y); g[7] = half_lo(ha.z); g[8] = half_hi(ha.z);
+      ajc = __uint_as_float(ha.w);
+      wb = hbb.y >> 16;
+      gb[0] = half_lo(hbb.x); gb[1] = half_hi(hbb.x); gb[2] = half_lo(hbb.y);
+    } else {
+      w = cur.w; wb = cur.wb; ajc = cur.aj;
+#pragma unroll
+      for (int q = 0; q < 9; q++) g[q] = cur.g[q];
+#pragma unroll
+      for (int q = 0; q < 3; q++) gb[q] = cur.gb[q];
     }
-    // operands of the output (FP64: loaded here, before the barrier)
-    T ajc = cur.aj, bc = cur.b, dvc = cur.dv;
-    if (!PF && out) {
-      ajc = ajo(t);
-      if (MODE >= 1) bc = b[t];
-      if (MODE == 2) dvc = dinv[t];
-    }
+    const T fi = tile_flux_i<T, ST_TC>(Pm, P, Q, c, r, w, g[0], g[1], g[2]);
+    const T fj = tile_flux_j<T, ST_TC>(Pm, P, Q, c, r, w, g[3], g[4], g[5]);
+    const T fk = tile_flux_k<T, ST_TC>(P, Q, c, r, w, g[6], g[7], g[8]);
+    T fj_lo = (T)0;
+    if (R * TW < 64)   // the wavefront of row 0 (whole wavefronts take one side)
+      fj_lo = tile_flux_j<T, ST_TC>(Pm, P, Q, c, 0, wb, gb[0], gb[1], gb[2]);
     const T xc = P[r * ST_TC + c];
     FJ[gk & 1][R][L] = fj;
-    if (gk + 2 <= k1) store_x(gk + 2, xn0, xn1);
+    store_x(gk + 2, xn);   // plane gk+2 (zeros past k1: not read)
     const T fi_lo = __shfl_up(fi, 1, TW);
     __syncthreads();
     if (R > 0) fj_lo = FJ[gk & 1][R - 1][L];
-    if (out) {
-      T res;
-      // MODE 2 with a colour: cells of the other (i+j+k) parity keep x
-      const bool keep = MODE == 2 && color >= 0 && ((gi + gj + gk) & 1) != color;
-      if (!(w & 1u)) {
-        const T xv = (T)x[t];
-        if (MODE == 0) res = xv;
-        else if (MODE == 1) res = bc - xv;
-        else res = keep ? xv : xv + omega * dvc * (bc - xv);
-      } else if (keep) {
-        res = xc;
-      } else {
-        T acc = 0;
-        acc += fi; acc -= fi_lo;
-        acc += fj; acc -= fj_lo;
-        acc += fk; acc -= fk_lo;
-        const T ax = -ajc * acc;
-        if (MODE == 0) res = ax;
-        else if (MODE == 1) res = bc - ax;
-        else res = xc + omega * dvc * (bc - ax);
-      }
-      y[t] = res;
-    }
+    // MODE 2 with a colour: cells of the other (i+j+k) parity keep x
+    const bool keep = MODE == 2 && color >= 0 && ((gi + gj + gk) & 1) != color;
+    T acc = 0;
+    acc += fi; acc -= fi_lo;
+    acc += fj; acc -= fj_lo;
+    acc += fk; acc -= fk_lo;
+    const bool fluid = w & 1u;
+    // identity rows take the cell's own x
+    const bool gh = ghost_i || (A.zper && (gk == 0 || gk == mz - 1));
+    const T xv = fluid ? xc : gh ? cur.xg : xc;
+    auto result = [&](T ax) -> T {
+      if constexpr (MODE == 0) return ax;
+      else if constexpr (MODE == 1) return cur.b - ax;
+      else return xv + omega * cur.dv * (cur.b - ax);
+    };
+    const T rf = result(-ajc * acc), rn = result(xv);
+    T res = fluid ? rf : rn;
+    if (MODE == 2) res = keep ? xv : res;
+    cv_bst<T>(By, res, oT, (unsigned)(gk - kb) * pl * (unsigned)sizeof(T));
     fk_lo = fk;
-    cur = nxt;
-    xn0 = xq0; xn1 = xq1;
+  };
+  StCell<T, HG> alt;
+  TX xalt[2];
+  for (int gk = k0;;) {
+    plane(gk, cur, alt, xn, xalt);
+    if (++gk >= k1) break;
+    plane(gk, alt, cur, xalt, xn);
+    if (++gk >= k1) break;
   }
 }
 
-template <class T, int MODE, int TY, bool PFB, bool HG = false, int TW = 64, class TX = T>
+template <class T, int MODE, int TY, bool HG = false, int TW = 64, class TX = T>
 __global__ void __launch_bounds__(TW * TY) k_stencil(OpV<T> A, const TX *__restrict__ x, const T *__restrict__ b,
                                                    T *__restrict__ y, const T *__restrict__ dinv, T omega, int kchunk,
                                                    int remap, int color) {
   int bx = blockIdx.x, by = blockIdx.y, bz = blockIdx.z;
   if (remap == 1) cv_xcd_tile(bx, by, bz);
   else if (remap > 1) cv_xcd_runs(remap, bx, by, bz);
-  stencil_tile<T, MODE, TY, PFB, HG, TW, TX>(A, x, b, y, dinv, omega, kchunk, bx, by, bz, color);
+  stencil_tile<T, MODE, TY, HG, TW, TX>(A, x, b, y, dinv, omega, kchunk, bx, by, bz, color);
 }
 
 // ------------------------------------------------------------------
@@ -1207,10 +1224,11 @@ static int stencil_rows() {
   if (!ty) ty = env_int(sizeof(T) == 8 ? "CV_STENCIL_ROWS64" : "CV_STENCIL_ROWS32", 4) == 8 ? 8 : 4;
   return ty;
 }
-static int stencil_pfb64() {
-  static int v = -1;
-  if (v < 0) v = env_int("CV_STENCIL_PFB64", 1) != 0;
-  return v;
+// k planes of a chunk such that the byte offsets of its widest operand (16
+// bytes a point) stay within 32 bits
+static int stencil_fit(int kc, const CvDims &d) {
+  const long most = (1L << 28) / ((long)d.mx * d.my) - 2;
+  return (int)std::max(1L, std::min((long)kc, most));
 }
 // tile order: 0 launch order, 1 one contiguous block range per XCD, R > 1
 // interleaved runs of R tiles; default (-1 here) runs of two rows of x-tiles,
@@ -1258,7 +1276,7 @@ template <class T, int MODE, class TX = T>
 static void stencil(cv_ctx *c, int l, const TX *x, const T *b, T *y, T omega = (T)0, int color = -1) {
   CvLevel &L = c->lev[l];
   OpV<T> A = opview<T>(c, l);
-  const int kc = stencil_kchunk(L.d.mz);
+  const int kc = stencil_fit(stencil_kchunk(L.d.mz), L.d);
   const int tw = stencil_tw(L.d.mx);
   const int ty = tw == 32 ? stencil_tw32_rows() : stencil_rows<T>();
   dim3 g((unsigned)((L.d.mx + tw - 2) / (tw - 1)), (unsigned)((L.d.my + ty - 1) / ty),
@@ -1267,50 +1285,23 @@ static void stencil(cv_ctx *c, int l, const TX *x, const T *b, T *y, T omega = (
   const bool hg = sizeof(T) == 4 && half_coef(c) && L.gh;
   CvProfScope ps(c, MODE == 0 ? CV_PROF_APPLY : CV_PROF_RESID, l, sizeof(T) == 4 ? 1 : 0,
                  (double)L.d.n * (stencil_bytes_pt<T>(MODE, hg) - (double)(sizeof(T) - sizeof(TX))));
-  const bool pfb = sizeof(T) == 4 || stencil_pfb64();
-  if (tw == 32) {
-    if constexpr (sizeof(T) == 4) {
-      if (hg) {
-        if (ty == 8)
-          hipLaunchKernelGGL((k_stencil<T, MODE, 8, true, true, 32, TX>), g, dim3(32, 8), 0, c->stream, A, x, b, y, A.dinv,
-                             omega, kc, remap, color);
-        else
-          hipLaunchKernelGGL((k_stencil<T, MODE, 4, true, true, 32, TX>), g, dim3(32, 4), 0, c->stream, A, x, b, y, A.dinv,
-                             omega, kc, remap, color);
-        return;
-      }
-    }
-    if (ty == 8)
-      hipLaunchKernelGGL((k_stencil<T, MODE, 8, true, false, 32, TX>), g, dim3(32, 8), 0, c->stream, A, x, b, y, A.dinv,
-                         omega, kc, remap, color);
-    else
-      hipLaunchKernelGGL((k_stencil<T, MODE, 4, true, false, 32, TX>), g, dim3(32, 4), 0, c->stream, A, x, b, y, A.dinv,
-                         omega, kc, remap, color);
-    return;
-  }
+#define ST_LAUNCH(TY, HG, TW)                                                                                       \
+  hipLaunchKernelGGL((k_stencil<T, MODE, TY, HG, TW, TX>), g, dim3(TW, TY), 0, c->stream, A, x, b, y, A.dinv, omega, kc, \
+                     remap, color)
   if constexpr (sizeof(T) == 4) {
     if (hg) {
-      if (ty == 4)
-        hipLaunchKernelGGL((k_stencil<T, MODE, 4, true, true, 64, TX>), g, dim3(64, 4), 0, c->stream, A, x, b, y, A.dinv, omega,
-                           kc, remap, color);
-      else
-        hipLaunchKernelGGL((k_stencil<T, MODE, 8, true, true, 64, TX>), g, dim3(64, 8), 0, c->stream, A, x, b, y, A.dinv, omega,
-                           kc, remap, color);
+      if (tw == 32 && ty == 8) ST_LAUNCH(8, true, 32);
+      else if (tw == 32) ST_LAUNCH(4, true, 32);
+      else if (ty == 8) ST_LAUNCH(8, true, 64);
+      else ST_LAUNCH(4, true, 64);
       return;
     }
   }
-  if (ty == 4 && pfb)
-    hipLaunchKernelGGL((k_stencil<T, MODE, 4, true, false, 64, TX>), g, dim3(64, 4), 0, c->stream, A, x, b, y, A.dinv, omega, kc, remap,
-                       color);
-  else if (ty == 4)
-    hipLaunchKernelGGL((k_stencil<T, MODE, 4, false, false, 64, TX>), g, dim3(64, 4), 0, c->stream, A, x, b, y, A.dinv, omega, kc, remap,
-                       color);
-  else if (pfb)
-    hipLaunchKernelGGL((k_stencil<T, MODE, 8, true, false, 64, TX>), g, dim3(64, 8), 0, c->stream, A, x, b, y, A.dinv, omega, kc, remap,
-                       color);
-  else
-    hipLaunchKernelGGL((k_stencil<T, MODE, 8, false, false, 64, TX>), g, dim3(64, 8), 0, c->stream, A, x, b, y, A.dinv, omega, kc, remap,
-                       color);
+  if (tw == 32 && ty == 8) ST_LAUNCH(8, false, 32);
+  else if (tw == 32) ST_LAUNCH(4, false, 32);
+  else if (ty == 8) ST_LAUNCH(8, false, 64);
+  else ST_LAUNCH(4, false, 64);
+#undef ST_LAUNCH
 }
 
 // sum of part[0..nb) -> dsc[slot] (device)

@@ -1,7 +1,10 @@
-"""The pressure solve's kernels where their tiles end: the y-line solve at the
-row counts where its chunks of 8, 16 and 32 rows fill, end and overflow.
+"""The pressure solve's kernels where their tiles end: the operator stencil
+on grids a cell short of, at and past its 31- and 63-cell rows, its rows in j
+and its k chunks, and the y-line solve at the row counts where its chunks of
+8, 16 and 32 rows fill, end and overflow.
 
-Tolerances: a line solve differs from a
+Tolerances: an operator apply differs from the oracle's assembled rows by
+rounding only (1e-13, as in the parity tests).  A line solve differs from a
 banded solve of the oracle's rows by the roundings of its own precision times
 the lines' conditioning."""
 import numpy as np
@@ -14,8 +17,31 @@ from oracle.pyoracle import from_case as oracle_case
 
 pytestmark = pytest.mark.gpu
 
+CHANNEL, BOX, OPEN = (7, 7, 1, 1, 7, 7), (1, 1, 1, 1, 1, 1), (7, 7, 1, 1, 5, 4)
+
+
 def rel(a, b):
     return float(np.linalg.norm(a - b) / max(np.linalg.norm(b), 1e-300))
+
+
+@pytest.mark.parametrize("cells,bctype,sphere", [
+    ((4, 4, 4), CHANNEL, None), ((28, 5, 9), BOX, None), ((29, 6, 10), CHANNEL, None), ((30, 7, 11), OPEN, None),
+    ((31, 9, 63), CHANNEL, None), ((60, 10, 64), BOX, (0.5, 0.5, 0.5, 0.5)), ((61, 11, 66), CHANNEL, None),
+    ((62, 13, 4), CHANNEL, None), ((93, 12, 12), OPEN, (0.5, 0.5, 0.5, 0.5)), ((5, 4, 194), CHANNEL, None),
+    ((6, 5, 201), BOX, None)])
+def test_operator_apply_at_tile_edges(cells, bctype, sphere):
+    case = cases.ChannelCase(cells=cells, amp=0.08, beta=1.5, sphere=sphere, re=300.0, seed=5, bctype=bctype, inlet=7)
+    u, _ = gpu_case(case, mglevels=1)
+    o, _ = oracle_case(case, nlev=1)
+    try:
+        o.poisson_lhs(0)
+        mx, my, mz = o.dims(0)[:3]
+        x = np.random.default_rng(11).standard_normal((mz, my, mx))
+        e = rel(u.PoissonApply(x, 0), o.matvec(0, x))
+        assert e < 1e-13, (cells, e)
+    finally:
+        u.close()
+        o.close()
 
 
 def _lines(o, case):
