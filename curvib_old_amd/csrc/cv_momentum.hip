@@ -60,16 +60,18 @@ inline unsigned nblk(long n) {
 // few iterations earlier and are still in the cache
 #define MARCH_TY 4
 #define MARCH_KC 16
-#define CV_MARCH(g)                                                                          \
+
+
+#define CV_MARCH(g, kc)                                                                      \
   const int i = blockIdx.x * 64 + threadIdx.x, j = blockIdx.y * MARCH_TY + threadIdx.y;      \
-  const int k0_ = blockIdx.z * MARCH_KC, k1_ = min(k0_ + MARCH_KC, (g).mz);                 \
+  const int k0_ = blockIdx.z * (kc), k1_ = min(k0_ + (kc), (g).mz);                         \
   if (i < (g).mx && j < (g).my)                                                              \
     for (int k = k0_; k < k1_; k++)
 
 // the same launch shape with the block given explicitly (batched launches)
-#define CV_MARCH_B(g, bx_, by_, bz_)                                                          \
+#define CV_MARCH_B(g, kc, bx_, by_, bz_)                                                      \
   const int i = (bx_) * 64 + threadIdx.x, j = (by_) * MARCH_TY + threadIdx.y;               \
-  const int k0_ = (bz_) * MARCH_KC, k1_ = min(k0_ + MARCH_KC, (g).mz);                      \
+  const int k0_ = (bz_) * (kc), k1_ = min(k0_ + (kc), (g).mz);                              \
   if (i < (g).mx && j < (g).my)                                                              \
     for (int k = k0_; k < k1_; k++)
 
@@ -79,9 +81,11 @@ struct GS {
 };
 #define GS_SELF GS{blockIdx.x * (long)blockDim.x + threadIdx.x, (long)gridDim.x * blockDim.x}
 
-inline dim3 march_grid(int mx, int my, int mz) {
-  return dim3((unsigned)((mx + 63) / 64), (unsigned)((my + MARCH_TY - 1) / MARCH_TY),
-              (unsigned)((mz + MARCH_KC - 1) / MARCH_KC));
+inline long march_columns(int mx, int my) {
+  return (long)((mx + 63) / 64) * ((my + MARCH_TY - 1) / MARCH_TY);
+}
+inline dim3 march_grid(int mx, int my, int mz, int kc) {
+  return dim3((unsigned)((mx + 63) / 64), (unsigned)((my + MARCH_TY - 1) / MARCH_TY), (unsigned)((mz + kc - 1) / kc));
 }
 #define MARCH_BLOCK dim3(64, MARCH_TY)
 
@@ -116,11 +120,10 @@ __device__ __forceinline__ void c2c_cell(G g, C3 uc, C3 csi, C3 eta, C3 zet, con
 // the k-march of the interior: the k-1 plane's zet and Ucont.z a cell reads
 // are the previous iteration's own values, carried in registers (a whole
 // plane of the XCD's blocks outgrows its L2 between the two reads)
-__device__ __forceinline__ void contra2cart_body(G g, C3 uc, C3 csi, C3 eta, C3 zet, const double *nv, V3 ucat, long n, int bx, int by, int bz) {
-  (void)n;
+__device__ __forceinline__ void contra2cart_body(G g, C3 uc, C3 csi, C3 eta, C3 zet, const double *nv, V3 ucat, int kc, int bx, int by, int bz) {
   const int i = bx * 64 + threadIdx.x, j = by * MARCH_TY + threadIdx.y;
   if (!(i > 0 && i < g.mx - 1 && j > 0 && j < g.my - 1)) return;
-  const int k0 = max(bz * MARCH_KC, 1), k1 = min(bz * MARCH_KC + MARCH_KC, g.mz - 1);
+  const int k0 = max(bz * kc, 1), k1 = min(bz * kc + kc, g.mz - 1);
   if (k0 >= k1) return;
   long t = g.at(i, j, k0 - 1);
   double zx = zet.x[t], zy = zet.y[t], zz = zet.z[t], wz = uc.z[t];
@@ -147,11 +150,11 @@ __device__ __forceinline__ void contra2cart_body(G g, C3 uc, C3 csi, C3 eta, C3 
 // with the same expression, the k-1 plane's is carried, so the bits are
 // those of the three passes in turn.
 __device__ __forceinline__ void rk_c2c_body(G g, double a, C3 uo, C3 r, V3 u, int wx, int wy, int wz, C3 csi, C3 eta,
-                                            C3 zet, const double *nv, V3 ucat, int bx, int by, int bz) {
+                                            C3 zet, const double *nv, V3 ucat, int kc, int bx, int by, int bz) {
   const int mx = g.mx, my = g.my, mz = g.mz;
   const int i = bx * 64 + threadIdx.x, j = by * MARCH_TY + threadIdx.y;
   if (!(i < mx && j < my)) return;
-  const int k0 = bz * MARCH_KC, k1 = min(k0 + MARCH_KC, mz);
+  const int k0 = bz * kc, k1 = min(k0 + kc, mz);
   auto ux = [&](long q, int ii) -> double {
     const double v = a * r.x[q] + uo.x[q];
     return (((wx & 1) && ii == 0) || ((wx & 2) && ii == mx - 2)) ? 0. : v;
@@ -191,10 +194,10 @@ __device__ __forceinline__ void rk_c2c_body(G g, double a, C3 uo, C3 r, V3 u, in
     zx = zx1; zy = zy1; zz = zz1; pz = vz;
   }
 }
-__global__ void k_contra2cart(G g, C3 uc, C3 csi, C3 eta, C3 zet, const double *nv, V3 ucat, long n) { contra2cart_body(g, uc, csi, eta, zet, nv, ucat, n, blockIdx.x, blockIdx.y, blockIdx.z); }
+__global__ void k_contra2cart(G g, C3 uc, C3 csi, C3 eta, C3 zet, const double *nv, V3 ucat, int kc) { contra2cart_body(g, uc, csi, eta, zet, nv, ucat, kc, blockIdx.x, blockIdx.y, blockIdx.z); }
 __global__ void __launch_bounds__(64 * MARCH_TY) k_rk_c2c(G g, double a, C3 uo, C3 r, V3 u, int wx, int wy, int wz, C3 csi,
-                                                         C3 eta, C3 zet, const double *nv, V3 ucat) {
-  rk_c2c_body(g, a, uo, r, u, wx, wy, wz, csi, eta, zet, nv, ucat, blockIdx.x, blockIdx.y, blockIdx.z);
+                                                         C3 eta, C3 zet, const double *nv, V3 ucat, int kc) {
+  rk_c2c_body(g, a, uo, r, u, wx, wy, wz, csi, eta, zet, nv, ucat, kc, blockIdx.x, blockIdx.y, blockIdx.z);
 }
 // Contra2Cart of the interior cells of one k plane
 __global__ void k_contra2cart_plane(G g, C3 uc, C3 csi, C3 eta, C3 zet, const double *nv, V3 ucat, int k) {
@@ -1205,16 +1208,15 @@ __device__ inline double ptan_v(int mode, double p0, double po, double pf, doubl
   return (a + b - c - d) * (lo || up ? 0.5 : 0.25);
 }
 
-__device__ __forceinline__ void ff1_faces_body(FFArgs A, V3 rhs, long n, int bx, int by, int bz) {
+__device__ __forceinline__ void ff1_faces_body(FFArgs A, V3 rhs, int kc, int bx, int by, int bz) {
   const G &g = A.g;
-  (void)n;
   // what the cell below (k-1) loaded that this cell reads again: its plane
   // k+1 points (this cell's p, pe, pn, pw, ps), its own p, pe, pn (this
   // cell's k-1 points), rct.z and nvert at k+1; valid after an interior cell
   bool have = false;
   double c_pt = 0., c_pet = 0., c_pnt = 0., c_ptw = 0., c_pts = 0., c_p0 = 0., c_pe = 0., c_pn = 0.;
   double c_rz = 0., c_nv = 0.;
-  CV_MARCH_B(g, bx, by, bz) {
+  CV_MARCH_B(g, kc, bx, by, bz) {
     const long t = g.at(i, j, k);
     if (!(i > 0 && i < g.mx - 1 && j > 0 && j < g.my - 1 && k > 0 && k < g.mz - 1)) { have = false; continue; }
     const double *p = A.p;
@@ -1276,7 +1278,7 @@ __device__ __forceinline__ void ff1_faces_body(FFArgs A, V3 rhs, long n, int bx,
     c_rz = rz1; c_nv = nvt;
   }
 }
-__global__ void __launch_bounds__(BS) k_ff1_faces(FFArgs A, V3 rhs, long n) { ff1_faces_body(A, rhs, n, blockIdx.x, blockIdx.y, blockIdx.z); }
+__global__ void __launch_bounds__(BS) k_ff1_faces(FFArgs A, V3 rhs, int kc) { ff1_faces_body(A, rhs, kc, blockIdx.x, blockIdx.y, blockIdx.z); }
 
 
 // the loop state after the main FormFunction1 sweep: the z-face values of
@@ -1397,9 +1399,9 @@ __global__ void k_rk_update(double a, C3 uo, C3 r, V3 u, long n) { rk_update_bod
 // at every storage point, then the zero set of the reference's interior and
 // boundary-plane masks (all of them only zero entries, so they commute)
 __global__ void __launch_bounds__(BS) k_calcrhs(G g, int bdf2, double idt, C3 u, C3 uo, C3 um, const double *nv,
-                                                V3 r, int yper) {
+                                                V3 r, int yper, int kc) {
   const int mx = g.mx, my = g.my, mz = g.mz, xper = g.xper, zper = g.zper;
-  CV_MARCH(g) {
+  CV_MARCH(g, kc) {
     const long t = g.at(i, j, k);
     double d0, d1, d2;
     if (bdf2) {
@@ -1488,14 +1490,16 @@ static G gview(cv_ctx *c) {
   g.sj = g.mx; g.sk = (long)g.mx * g.my;
   return g;
 }
+static int march_kc(const CvDims &d) { return cv_march_kchunk(march_columns(d.mx, d.my), d.mz, MARCH_KC, MARCH_BLOCKS); }
 static V3 v3(double *const a[3]) { return V3{a[0], a[1], a[2]}; }
 static C3 c3(double *const a[3]) { return C3{a[0], a[1], a[2]}; }
 
 int cv_contra2cart_dev(cv_ctx *c) {
   CvLevel &F = c->lev[c->nlev - 1];
   CvMetrics &M = c->m;
-  hipLaunchKernelGGL(k_contra2cart, march_grid(F.d.mx, F.d.my, F.d.mz), MARCH_BLOCK, 0, c->stream, gview(c), c3(c->ucont), c3(M.csi),
-                     c3(M.eta), c3(M.zet), (const double *)F.nvert, v3(c->ucat), F.d.n);
+  const int kc = march_kc(F.d);
+  hipLaunchKernelGGL(k_contra2cart, march_grid(F.d.mx, F.d.my, F.d.mz, kc), MARCH_BLOCK, 0, c->stream, gview(c),
+                     c3(c->ucont), c3(M.csi), c3(M.eta), c3(M.zet), (const double *)F.nvert, v3(c->ucat), kc);
   CV_CHECK(hipGetLastError());
   return CV_OK;
 }
@@ -1753,14 +1757,16 @@ static int rc_rows() {
   return ty;
 }
 
-// k planes per face-flux block (CV_RC_KC)
-static int rc_kchunk() {
-  static int kc = 0;
-  if (!kc) {
+// k planes per face-flux block (CV_RC_KC, else by the number of its (i, j)
+// tiles, as the other marches)
+static long rc_columns(int mx, int my, int ty) { return (long)((mx + 62) / 63) * ((my - 1 + ty - 2) / (ty - 1)); }
+static int rc_kchunk(long columns, int mz) {
+  static int kc = -1;
+  if (kc < 0) {
     const char *e = getenv("CV_RC_KC");
-    kc = e ? std::max(1, atoi(e)) : RC_KC;
+    kc = e ? std::max(1, atoi(e)) : 0;
   }
-  return kc;
+  return kc ? kc : cv_march_kchunk(columns, mz, RC_KC, RC_BLOCKS);
 }
 
 // face-flux pass variant (CV_RC_KERNEL: 1 LDS-tiled, 0 global gathers),
@@ -1803,7 +1809,7 @@ int cv_ff1_dev(cv_ctx *c) {
     // ucont, ucat, nvert, rct out
     CvProfScope ps(c, CV_PROF_RCT, c->nlev - 1, 0, (double)F.d.n * 8.0 * (30 + 10 + 3 + 3 + 1 + 3));
     const int ty = rc_rows(), tiled = rc_kernel();
-    const int kc = rc_kchunk();
+    const int kc = rc_kchunk(rc_columns(F.d.mx, F.d.my, ty), F.d.mz);
     const dim3 grid((unsigned)((F.d.mx + 62) / 63), (unsigned)((F.d.my - 1 + ty - 2) / (ty - 1)),
                     (unsigned)((F.d.mz + kc - 1) / kc));
     auto kern = tiled ? (ty == 8 ? k_rc_tiled<8> : k_rc_tiled<4>) : (ty == 8 ? k_rc_fused<8> : k_rc_fused<4>);
@@ -1816,7 +1822,8 @@ int cv_ff1_dev(cv_ctx *c) {
   {
     // algorithmic bytes per point: p, rct, 9 face coefficients, nvert, Rhs out, the operator word
     CvProfScope ps(c, CV_PROF_FF1, c->nlev - 1, 0, (double)F.d.n * (8.0 * (1 + 3 + 9 + 1 + 3) + 4.0));
-    hipLaunchKernelGGL(k_ff1_faces, march_grid(F.d.mx, F.d.my, F.d.mz), MARCH_BLOCK, 0, c->stream, A, v3(c->rhs), F.d.n);
+    const int kc = march_kc(F.d);
+    hipLaunchKernelGGL(k_ff1_faces, march_grid(F.d.mx, F.d.my, F.d.mz, kc), MARCH_BLOCK, 0, c->stream, A, v3(c->rhs), kc);
   }
   if (F.d.xper || F.d.zper) {
     long nf = (F.d.xper ? (long)(A.g.my - 2) * (A.g.mz - 2) : 0) + (F.d.zper ? (long)(A.g.my - 2) * (A.g.mx - 2) : 0);
@@ -1846,9 +1853,10 @@ int cv_rk_dev(cv_ctx *c) {
     double a = alfa[s] * c->dt * c->st;
     if (fused) {
       CvMetrics &M = c->m;
-      hipLaunchKernelGGL(k_rk_c2c, march_grid(F.d.mx, F.d.my, F.d.mz), MARCH_BLOCK, 0, c->stream, g, a, c3(c->ucont_o),
+      const int kc = march_kc(F.d);
+      hipLaunchKernelGGL(k_rk_c2c, march_grid(F.d.mx, F.d.my, F.d.mz, kc), MARCH_BLOCK, 0, c->stream, g, a, c3(c->ucont_o),
                          c3(c->rhs), v3(c->ucont), wx, wy, wz, c3(M.csi), c3(M.eta), c3(M.zet), (const double *)F.nvert,
-                         v3(c->ucat));
+                         v3(c->ucat), kc);
       if ((rc = cv_ghost_update(c, 1, false))) return rc;
       continue;
     }
@@ -1868,9 +1876,10 @@ int cv_calcrhs_dev(cv_ctx *c) {
   G g = gview(c);
   int rc = cv_ff1_dev(c);
   if (rc) return rc;
-  hipLaunchKernelGGL(k_calcrhs, march_grid(F.d.mx, F.d.my, F.d.mz), MARCH_BLOCK, 0, c->stream, g,
+  const int kc = march_kc(F.d);
+  hipLaunchKernelGGL(k_calcrhs, march_grid(F.d.mx, F.d.my, F.d.mz, kc), MARCH_BLOCK, 0, c->stream, g,
                      c->steps_done > 0 ? 1 : 0, -1. / c->dt, c3(c->ucont), c3(c->ucont_o), c3(c->ucont_rm1),
-                     (const double *)F.nvert, v3(c->rhs), c->bctype[2] == 7 ? 1 : 0);
+                     (const double *)F.nvert, v3(c->rhs), c->bctype[2] == 7 ? 1 : 0, kc);
   CV_CHECK(hipGetLastError());
   return CV_OK;
 }
@@ -2119,7 +2128,7 @@ struct MCase {
   double nu, dt, st;
   int wx, wy, wz;           // wall masks of the i, j and k faces (wall-normal flux reset)
   long n;
-  int mgx, mgy, mgz;        // k-marching blocks
+  int mgx, mgy, mgz, mkc;   // k-marching blocks and their k planes
   int rgx, rgy, rgz, rkc;   // face-flux tiles (8 rows) and their k planes
   int nvb, npb;             // blocks of an elementwise and of a plane pass
 };
@@ -2150,7 +2159,7 @@ __global__ void kbm_vec3(MB_ARGS, int which) {
 __global__ void __launch_bounds__(64 * MARCH_TY) kbm_contra2cart(MB_ARGS) {
   MB_HEAD
   const int bx = lb % C.mgx, by = (lb / C.mgx) % C.mgy, bz = lb / (C.mgx * C.mgy);
-  contra2cart_body(C.g, mc3(C.uc), C.csi, C.eta, C.zet, C.nv, mv3(C.uca), C.n, bx, by, bz);
+  contra2cart_body(C.g, mc3(C.uc), C.csi, C.eta, C.zet, C.nv, mv3(C.uca), C.mkc, bx, by, bz);
 }
 
 __global__ void kbm_wall_ghost(MB_ARGS, int full) {
@@ -2191,7 +2200,7 @@ __global__ void kbm_rct_periodic(MB_ARGS) {
 __global__ void __launch_bounds__(BS) kbm_ff1_faces(MB_ARGS) {
   MB_HEAD
   const int bx = lb % C.mgx, by = (lb / C.mgx) % C.mgy, bz = lb / (C.mgx * C.mgy);
-  ff1_faces_body(C.ff, mv3(C.rhs), C.n, bx, by, bz);
+  ff1_faces_body(C.ff, mv3(C.rhs), C.mkc, bx, by, bz);
 }
 
 __global__ void kbm_ff1_periodic(MB_ARGS) {
@@ -2215,8 +2224,8 @@ __global__ void __launch_bounds__(64 * MARCH_TY) kbm_rk_c2c(MB_ARGS, double alfa
   MB_HEAD
   const double a = alfa * C.dt * C.st;
   const int bx = lb % C.mgx, by = (lb / C.mgx) % C.mgy, bz = lb / (C.mgx * C.mgy);
-  rk_c2c_body(C.g, a, mc3(C.uo), mc3(C.rhs), mv3(C.uc), C.wx, C.wy, C.wz, C.csi, C.eta, C.zet, C.nv, mv3(C.uca), bx, by,
-              bz);
+  rk_c2c_body(C.g, a, mc3(C.uo), mc3(C.rhs), mv3(C.uc), C.wx, C.wy, C.wz, C.csi, C.eta, C.zet, C.nv, mv3(C.uca), C.mkc,
+              bx, by, bz);
 }
 
 }  // namespace
@@ -2294,6 +2303,16 @@ int cv_mom_batch_create(cv_ctx *const *cases, int n, hipStream_t s, CvMomBatch *
   std::vector<MCase> hc(n);
   std::vector<uint32_t> tabs;
   std::vector<int> cnt[5];
+  // the cases share every launch, so the k chunks follow their summed tiles
+  long mcol = 0, rcol = 0;
+  int mzmax = 0;
+  for (int c = 0; c < n; c++) {
+    const CvDims &d = cases[c]->lev[cases[c]->nlev - 1].d;
+    mcol += march_columns(d.mx, d.my);
+    rcol += rc_columns(d.mx, d.my, 8);
+    mzmax = std::max(mzmax, d.mz);
+  }
+  const int mkc = cv_march_kchunk(mcol, mzmax, MARCH_KC, MARCH_BLOCKS), rkc = rc_kchunk(rcol, mzmax);
   for (int c = 0; c < n; c++) {
     cv_ctx *x = cases[c];
     CvLevel &F = x->lev[x->nlev - 1];
@@ -2320,9 +2339,10 @@ int cv_mom_batch_create(cv_ctx *const *cases, int n, hipStream_t s, CvMomBatch *
     m.wy = wall_mask(x->bctype[2], x->bctype[3]);
     m.wz = wall_mask(x->bctype[4], x->bctype[5]);
     m.n = F.d.n;
-    const dim3 mg = march_grid(F.d.mx, F.d.my, F.d.mz);
+    m.mkc = mkc;
+    const dim3 mg = march_grid(F.d.mx, F.d.my, F.d.mz, m.mkc);
     m.mgx = (int)mg.x; m.mgy = (int)mg.y; m.mgz = (int)mg.z;
-    m.rkc = rc_kchunk();
+    m.rkc = rkc;
     m.rgx = (F.d.mx + 62) / 63; m.rgy = (F.d.my - 1 + 6) / 7; m.rgz = (F.d.mz + m.rkc - 1) / m.rkc;
     m.nvb = (int)std::min<long>((F.d.n + BS - 1) / BS, 1024);
     const long planes = (long)F.d.my * F.d.mz + (long)F.d.mx * F.d.mz + (long)F.d.mx * F.d.my;

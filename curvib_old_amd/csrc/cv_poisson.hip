@@ -2181,17 +2181,17 @@ __device__ __forceinline__ static void projection_body(Idx I, int xper, int zper
 }
 
 
-// The projection as a k-march (64 x PJ_TY threads walk PJ_KC planes): the
+// The projection as a k-march (64 x PJ_TY threads walk kc planes): the
 // same faces as projection_body, each cell taking 8 of its phi points and
 // its nvert from the cell below it in registers
 #define PJ_TY 4
 #define PJ_KC 16
 __global__ static void __launch_bounds__(64 * PJ_TY)
     k_projection_march(Idx I, int xper, int zper, const double *phi, const double *nv, const uint32_t *fl, FaceMet Mi,
-                       FaceMet Mj, FaceMet Mk, double *ux, double *uy, double *uz, double dt, double st) {
+                       FaceMet Mj, FaceMet Mk, double *ux, double *uy, double *uz, double dt, double st, int kc) {
   const int i = blockIdx.x * 64 + threadIdx.x, j = blockIdx.y * PJ_TY + threadIdx.y;
   if (i >= I.mx || j >= I.my) return;
-  const int k0 = blockIdx.z * PJ_KC, k1 = min(k0 + PJ_KC, I.mz);
+  const int k0 = blockIdx.z * kc, k1 = min(k0 + kc, I.mz);
   const int i_end = xper ? I.mx - 1 : I.mx - 2, j_end = I.my - 2, k_end = zper ? I.mz - 1 : I.mz - 2;
   const bool iin = i > 0 && i < I.mx - 1, jin = j > 0 && j < I.my - 1;
   const long sj = (long)I.mx, sk = (long)I.mx * I.my;
@@ -2225,11 +2225,12 @@ int cv_projection_dev(cv_ctx *c) {
   FaceMet Mi{{F.g[0], F.g[1], F.g[2]}};
   FaceMet Mj{{F.g[3], F.g[4], F.g[5]}};
   FaceMet Mk{{F.g[6], F.g[7], F.g[8]}};
-  const dim3 grid((unsigned)((F.d.mx + 63) / 64), (unsigned)((F.d.my + PJ_TY - 1) / PJ_TY),
-                  (unsigned)((F.d.mz + PJ_KC - 1) / PJ_KC));
+  const unsigned gx = (unsigned)((F.d.mx + 63) / 64), gy = (unsigned)((F.d.my + PJ_TY - 1) / PJ_TY);
+  const int kc = cv_march_kchunk((long)gx * gy, F.d.mz, PJ_KC, MARCH_BLOCKS);
+  const dim3 grid(gx, gy, (unsigned)((F.d.mz + kc - 1) / kc));
   hipLaunchKernelGGL(k_projection_march, grid, dim3(64, PJ_TY), 0, c->stream, idx_of(F), F.d.xper, F.d.zper,
                      (const double *)c->phi, (const double *)F.nvert, (const uint32_t *)F.flags, Mi, Mj, Mk,
-                     c->ucont[0], c->ucont[1], c->ucont[2], c->dt, c->st);
+                     c->ucont[0], c->ucont[1], c->ucont[2], c->dt, c->st, kc);
   CV_CHECK(hipGetLastError());
   int rc = cv_contra2cart_dev(c);
   if (rc) return rc;
@@ -2292,7 +2293,7 @@ __device__ __forceinline__ void divmax_block(Idx I, const double *ux, const doub
 }
 
 // divmax_block_s<1> as k-marches: block b takes tiles b, b + nb, ... of 64 x
-// DV_TY columns by DV_KC planes, and each column's cell takes uz and two
+// DV_TY columns by kc planes, and each column's cell takes uz and two
 // nvert planes from the cell below it.  Every point is visited once, and
 // the maximum with its first index does not depend on the visiting order,
 // so the partials reduce to the same (value, index) as the flat pass
@@ -2300,11 +2301,11 @@ __device__ __forceinline__ void divmax_block(Idx I, const double *ux, const doub
 #define DV_KC 16
 __global__ static void __launch_bounds__(64 * DV_TY)
     k_divmax_march(Idx I, const double *ux, const double *uy, const double *uz, const double *aj, const double *nv,
-                   double *pv, double *pi) {
+                   double *pv, double *pi, int kc) {
   static_assert(64 * DV_TY == BS, "one reduction slot per thread");
   __shared__ double sv[BS];
   __shared__ long si[BS];
-  const int tx = (I.mx + 63) / 64, ty = (I.my + DV_TY - 1) / DV_TY, tz = (I.mz + DV_KC - 1) / DV_KC;
+  const int tx = (I.mx + 63) / 64, ty = (I.my + DV_TY - 1) / DV_TY, tz = (I.mz + kc - 1) / kc;
   const long ntile = (long)tx * ty * tz;
   const long sj = I.mx, sk = (long)I.mx * I.my;
   double best = -1.0;
@@ -2313,7 +2314,7 @@ __global__ static void __launch_bounds__(64 * DV_TY)
     const int bx = (int)(tb % tx), by = (int)((tb / tx) % ty), bz = (int)(tb / ((long)tx * ty));
     const int i = bx * 64 + threadIdx.x, j = by * DV_TY + threadIdx.y;
     if (i >= I.mx || j >= I.my) continue;
-    const int k0 = bz * DV_KC, k1 = min(k0 + DV_KC, I.mz);
+    const int k0 = bz * kc, k1 = min(k0 + kc, I.mz);
     const bool ij = i > 0 && i < I.mx - 1 && j > 0 && j < I.my - 1;
     bool have = false;
     double c_uz = 0., c_n0 = 0., c_nt = 0.;   // the cell below's uz[t], nv[t], nv[t + sk]
@@ -2351,9 +2352,10 @@ __global__ static void __launch_bounds__(64 * DV_TY)
 int cv_divergence_dev(cv_ctx *c, double *maxdiv, long *idx) {
   CvLevel &F = c->lev[c->nlev - 1];
   const int nb = CV_RED_GRID;
+  const int kc = cv_march_kchunk((long)((F.d.mx + 63) / 64) * ((F.d.my + DV_TY - 1) / DV_TY), F.d.mz, DV_KC, nb);
   hipLaunchKernelGGL(k_divmax_march, dim3(nb), dim3(64, DV_TY), 0, c->stream, idx_of(F), (const double *)c->ucont[0],
                      (const double *)c->ucont[1], (const double *)c->ucont[2], (const double *)F.aj,
-                     (const double *)F.nvert, c->part, c->part + nb);
+                     (const double *)F.nvert, c->part, c->part + nb, kc);
   std::vector<double> hv(2 * nb);
   CV_CHECK(hipMemcpyAsync(hv.data(), c->part, 2 * nb * sizeof(double), hipMemcpyDeviceToHost, c->stream));
   CV_CHECK(hipStreamSynchronize(c->stream));
