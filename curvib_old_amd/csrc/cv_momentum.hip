@@ -290,36 +290,51 @@ __device__ __forceinline__ void periodic_planes_body(G g, V3 u, double *p, doubl
 __global__ void k_periodic_planes(G g, V3 u, double *p, double *nv) { periodic_planes_body(g, u, p, nv, GS_SELF); }
 
 
-// edge averages, twelve sequential sub-sweeps (bcs.c:5440-5566); one block
+// edge averages (bcs.c:5440-5566: twelve sub-sweeps in turn, along the edges
+// of the k planes, then the four edges along k); one block.  Between its ends
+// an edge reads face ghosts only, so the twelve run together; an edge along
+// k comes last at the corners and reads points beside them that the k-plane
+// edges just wrote, and no sub-sweep reads a corner.  So two rounds leave the
+// values of the twelve in turn (9 against 19 us at 32 cells an axis, where
+// each of the twelve waited for its own loads)
 __device__ __forceinline__ void edge_average_body(G g, V3 u, double *p) {
   const int mx = g.mx, my = g.my, mz = g.mz;
-  for (int sb = 0; sb < 12; sb++) {
-    int len;
-    int side = (sb < 8) ? (sb / 4) : ((sb - 8) / 2);
-    if (sb < 8) len = ((sb % 4) < 2) ? my : mx;
-    else len = mz;
-    for (int q = threadIdx.x; q < len; q += blockDim.x) {
-      long d, a, b;
-      if (sb < 8) {
-        int k = side ? mz - 1 : 0, kn = side ? mz - 2 : 1;
-        switch (sb % 4) {
-          case 0: d = g.at(0, q, k); a = g.at(0, q, kn); b = g.at(1, q, k); break;
-          case 1: d = g.at(mx - 1, q, k); a = g.at(mx - 1, q, kn); b = g.at(mx - 2, q, k); break;
-          case 2: d = g.at(q, 0, k); a = g.at(q, 0, kn); b = g.at(q, 1, k); break;
-          default: d = g.at(q, my - 1, k); a = g.at(q, my - 1, kn); b = g.at(q, my - 2, k); break;
-        }
-      } else {
-        int j = side ? my - 1 : 0, jn = side ? my - 2 : 1;
-        if ((sb - 8) % 2 == 0) { d = g.at(0, j, q); a = g.at(0, jn, q); b = g.at(1, j, q); }
-        else { d = g.at(mx - 1, j, q); a = g.at(mx - 1, jn, q); b = g.at(mx - 2, j, q); }
+  // point q of edge sb: 0-7 on the k planes (k side sb / 4), 8-11 along k
+  auto point = [&](int sb, int q) {
+    long d, a, b;
+    if (sb < 8) {
+      const int k = sb / 4 ? mz - 1 : 0, kn = sb / 4 ? mz - 2 : 1;
+      switch (sb % 4) {
+        case 0: d = g.at(0, q, k); a = g.at(0, q, kn); b = g.at(1, q, k); break;
+        case 1: d = g.at(mx - 1, q, k); a = g.at(mx - 1, q, kn); b = g.at(mx - 2, q, k); break;
+        case 2: d = g.at(q, 0, k); a = g.at(q, 0, kn); b = g.at(q, 1, k); break;
+        default: d = g.at(q, my - 1, k); a = g.at(q, my - 1, kn); b = g.at(q, my - 2, k); break;
       }
-      u.x[d] = 0.5 * (u.x[a] + u.x[b]);
-      u.y[d] = 0.5 * (u.y[a] + u.y[b]);
-      u.z[d] = 0.5 * (u.z[a] + u.z[b]);
-      if (p) p[d] = 0.5 * (p[a] + p[b]);
+    } else {
+      const int side = (sb - 8) / 2, j = side ? my - 1 : 0, jn = side ? my - 2 : 1;
+      if ((sb - 8) % 2 == 0) { d = g.at(0, j, q); a = g.at(0, jn, q); b = g.at(1, j, q); }
+      else { d = g.at(mx - 1, j, q); a = g.at(mx - 1, jn, q); b = g.at(mx - 2, j, q); }
     }
-    __syncthreads();
+    const double x = 0.5 * (u.x[a] + u.x[b]), y = 0.5 * (u.y[a] + u.y[b]), z = 0.5 * (u.z[a] + u.z[b]);
+    const double w = p ? 0.5 * (p[a] + p[b]) : 0.0;
+    u.x[d] = x; u.y[d] = y; u.z[d] = z;
+    if (p) p[d] = w;
+  };
+  const int ly = my - 2, lx = mx - 2, lz = mz - 2, n = 4 * (ly + lx + lz);   // edges without their ends
+  for (int t = threadIdx.x; t < n; t += blockDim.x) {
+    if (t < 4 * ly) {
+      const int e = t / ly;                       // 0, 1 on k = 0; 2, 3 on k = mz-1
+      point(4 * (e / 2) + e % 2, 1 + t - e * ly);
+    } else if (t < 4 * (ly + lx)) {
+      const int r = t - 4 * ly, e = r / lx;
+      point(4 * (e / 2) + 2 + e % 2, 1 + r - e * lx);
+    } else {
+      const int r = t - 4 * (ly + lx), e = r / lz;
+      point(8 + e, 1 + r - e * lz);
+    }
   }
+  __syncthreads();
+  if (threadIdx.x < 8) point(8 + threadIdx.x / 2, threadIdx.x % 2 ? mz - 1 : 0);
 }
 __global__ void k_edge_average(G g, V3 u, double *p) { edge_average_body(g, u, p); }
 
