@@ -137,6 +137,19 @@ __global__ void __launch_bounds__(1024) kb_yline(BK_ARGS, int d, int sr, T omega
                             HL ? (T)(omega * A.ysc) : omega, zg, lb, A.yh, A.yc);
 }
 
+// the coarse sweeps and the nullspace rule of the cases whose coarsest level
+// is depth d, one work-group a case
+template <class T, bool HG, int CS, int FPT>
+__global__ void __launch_bounds__(COARSE_NT) kb_coarse(const BCase *__restrict__ cs, unsigned long long pm,
+                                                       const BCtl *__restrict__ ctl, int d, T omega, int nsweep) {
+  const int c = blockIdx.x;
+  if (!(((pm & ctl->act) >> c) & 1ull)) return;
+  const BCase &C = cs[c];
+  const OpV<T> A = bop<T>(C, d);
+  coarse_body<T, HG, CS, FPT>(A, bvec<T>(C, d, BB, 0), bvec<T>(C, d, BX, ctl->jj), HG ? (T)(omega * A.ysc) : omega, nsweep,
+                              C.lev[d].inv_nf, C.lev[d].nrd, (T *)coarse_lds);
+}
+
 // r of depth d -> b of depth d+1 (block table of depth d+1)
 template <class T>
 __global__ void kb_restrict(BK_ARGS, int d) {
@@ -537,6 +550,36 @@ static void b_nullspace(cv_batch *B, int d, unsigned long long pm, int sx) {
 
 #include "cv_batch_legs.h"
 
+// the coarse solves of depth d as one work-group a case, one launch per rows
+// per thread of the line solve (8, 16), when every case bottoming out there
+// fits: beside the launches of one that does not, the kernel would only add
+// its time.  False where the launches run
+template <class T>
+static bool b_coarse(cv_batch *B, int d, unsigned long long co) {
+  const bool hg = sizeof(T) == 4 && B->opt.precision == CV_MIXED16;
+  unsigned long long m[2] = {0, 0};
+  int faces[2] = {0, 0}, lds[2] = {0, 0};
+  for (int c = 0; c < B->n; c++) {
+    if (!(co >> c & 1ull)) continue;
+    const CvDims &D = B->cs[c]->lev[B->cs[c]->nlev - 1 - d].d;
+    if (!coarse_fits<T>(D, true)) return false;
+    const CoDims K(D.mx, D.my, D.mz);
+    const int rows = coarse_rows(D, true), g = rows == 8 ? 0 : 1;
+    m[g] |= 1ull << c;
+    faces[g] = std::max(faces[g], K.faces());
+    lds[g] = std::max(lds[g], K.lds(rows) * (int)sizeof(T));
+  }
+  for (int g = 0; g < 2; g++)
+    if (m[g])
+      coarse_dispatch<T>(hg, g == 0 ? 8 : 16, faces[g], [&](auto h, auto rows, auto fpt) {
+        if constexpr (rows() > 0)
+          hipLaunchKernelGGL((kb_coarse<T, h(), rows(), fpt()>), dim3((unsigned)B->n), dim3(COARSE_NT), lds[g], B->stream,
+                             (const BCase *)B->dcases, m[g], (const BCtl *)B->dctl, d, (T)B->opt.omega,
+                             B->opt.coarse_sweeps);
+      });
+  return true;
+}
+
 // the V-cycle of depth d for every case that has it; the cases whose
 // coarsest level is at depth d run the coarse sweeps and the nullspace rule
 template <class T>
@@ -547,7 +590,7 @@ static void b_vcycle(cv_batch *B, int d) {
   }
   const cv_solver_opts &o = B->opt;
   const T om = (T)o.omega;
-  const unsigned long long in = B->inner[d], co = B->coarse[d];
+  const unsigned long long in = B->inner[d], co = b_coarse<T>(B, d, B->coarse[d]) ? 0 : B->coarse[d];
   const int npre = o.pre_sweeps, npost = o.post_sweeps, nco = o.coarse_sweeps;
   const unsigned long long z = (npre == 0 ? in : 0) | (nco == 0 ? co : 0);
   if (z) b_zero<T>(B, d, z, BX);

@@ -1169,6 +1169,8 @@ static int nred(long n) {
   return (int)b;
 }
 
+#include "cv_coarse.h"
+
 // k extent of one stencil block (tunable through CV_STENCIL_KCHUNK)
 static int stencil_kchunk(int mz) {
   static int kc = -1;
@@ -1597,10 +1599,33 @@ static void smooth(cv_ctx *c, MgVecs<T> &v, int l, int nsweep, bool zero_guess) 
   }
 }
 
+// the coarse sweeps and the nullspace rule of level 0 in one work-group;
+// false where they stay launches (a large level, the red-black smoother, a
+// kernel timed on that level)
+template <class T>
+static bool coarse_solve(cv_ctx *c, MgVecs<T> &v) {
+  CvLevel &L = c->lev[0];
+  const bool line = c->opt.smoother == CV_SMOOTH_YLINE;
+  const bool hg = sizeof(T) == 4 && half_coef(c) && L.gh;
+  if (c->opt.smoother == CV_SMOOTH_RB || !coarse_fits<T>(L.d, line)) return false;
+  if (c->prof.kind != CV_PROF_NONE && (c->prof.level == 0 || c->nlev == 1)) return false;
+  const OpV<T> A = opview<T>(c, 0);
+  const T om = (T)c->opt.omega * (line && hg ? (T)A.ysc : (T)1);
+  const CoDims D(L.d.mx, L.d.my, L.d.mz);
+  const double inv = c->nfluid[0] > 0 ? 1.0 / c->nfluid[0] : 0.0;
+  const int rows = coarse_rows(L.d, line);
+  coarse_dispatch<T>(hg, rows, D.faces(), [&](auto hgc, auto cs, auto fpt) {
+    hipLaunchKernelGGL((k_coarse<T, hgc(), cs(), fpt()>), dim3(1), dim3(COARSE_NT), D.lds(rows) * sizeof(T), c->stream, A,
+                       (const T *)v.b[0], v.x[0], om, c->opt.coarse_sweeps, inv, nred(L.d.n));
+  });
+  return true;
+}
+
 template <class T>
 static void vcycle(cv_ctx *c, MgVecs<T> &v, int l) {
   CvLevel &L = c->lev[l];
   const long n = L.d.n;
+  if (l == 0 && coarse_solve<T>(c, v)) return;
   if (l == 0) {
     smooth<T>(c, v, 0, c->opt.coarse_sweeps, true);
     nullspace_dev<T>(c, 0, v.x[0]);

@@ -3,6 +3,8 @@ on grids a cell short of, at and past its 31- and 63-cell rows, its rows in j
 and its k chunks, and the y-line solve at the row counts where its chunks of
 8, 16 and 32 rows fill, end and overflow.
 
+The coarsest level in one work-group against the launches it replaces.
+
 Tolerances: an operator apply differs from the oracle's assembled rows by
 rounding only (1e-13, as in the parity tests).  A line solve differs from a
 banded solve of the oracle's rows by the roundings of its own precision times
@@ -100,3 +102,31 @@ def test_line_solve_at_chunk_edges(rows):
         # three roundings a row, amplified by the lines' conditioning
         print(f"rows {rows} {prec}: {e:.2e}, conditioning {cond:.1f}", flush=True)
         assert e < 3 * eps * cond, (rows, prec, e, cond)
+
+
+@pytest.mark.parametrize("cells,bctype,sphere", [
+    ((3, 4, 3), CHANNEL, None), ((8, 8, 8), BOX, (0.5, 0.5, 0.5, 0.5)), ((4, 32, 4), CHANNEL, None),
+    ((5, 33, 7), OPEN, None), ((12, 8, 20), CHANNEL, (0.5, 0.5, 0.5, 0.5)), ((3, 128, 3), CHANNEL, None),
+    ((3, 129, 4), BOX, None), ((3, 200, 3), CHANNEL, None), ((16, 5, 16), CHANNEL, None), ((31, 4, 14), OPEN, None)])
+def test_coarsest_level_in_one_work_group_keeps_the_bits(cells, bctype, sphere):
+    """The coarsest level's sweeps and nullspace rule as one work-group against
+    the same as launches, which run where a kernel of that level is timed: the
+    same phi bit for bit, up to the sizes where a thread takes seven faces."""
+    case = cases.ChannelCase(cells=cells, amp=0.05, beta=1.0, sphere=sphere, re=300.0, seed=8, dt=2e-4, bctype=bctype,
+                             inlet=7)
+    u, _ = gpu_case(case, mglevels=1)
+    try:
+        for prec in ("fp64", "mixed", "mixed16"):
+            for smoother, omega in (("yline", 0.9), ("jacobi", 0.8)):
+                u.set_solver(precision=prec, smoother=smoother, omega=omega, coarse_sweeps=7, rtol=1e-8, max_it=8)
+                u.prof_select("none")
+                a = u.PoissonSolver_MG(allow_unconverged=True)
+                phi = u.get("phi")
+                u.prof_select("resid", level=0)
+                b = u.PoissonSolver_MG(allow_unconverged=True)
+                n = u.prof_read()[0]
+                assert n >= 6, (cells, prec, smoother, n)       # the launches did run
+                assert a["ksp_its"] == b["ksp_its"] and a["ksp_rnorm"] == b["ksp_rnorm"], (cells, prec, smoother, a, b)
+                assert np.isfinite(phi).all() and np.array_equal(phi, u.get("phi")), (cells, prec, smoother)
+    finally:
+        u.close()
