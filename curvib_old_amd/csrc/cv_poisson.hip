@@ -2277,12 +2277,9 @@ __host__ __device__ inline bool div_beats(double v2, long i2, double v1, long i1
 // block bid of nb: the largest |div| of its grid-stride share and its first
 // index (ties go to the smaller index, so the result does not depend on
 // the partition)
-// S: element stride of the flux components (1: planar arrays, 3: the
-// interleaved Cmpnts of the DMDA layout, ux = u, uy = u + 1, uz = u + 2)
-template <int S>
-__device__ __forceinline__ void divmax_block_s(Idx I, const double *ux, const double *uy, const double *uz,
-                                               const double *aj, const double *nv, long n, double *pv, double *pi,
-                                               int bid, int nb) {
+__device__ __forceinline__ void divmax_block(Idx I, const double *ux, const double *uy, const double *uz,
+                                             const double *aj, const double *nv, long n, double *pv, double *pi,
+                                             int bid, int nb) {
   __shared__ double sv[BS];
   __shared__ long si[BS];
   double best = -1.0;
@@ -2293,7 +2290,7 @@ __device__ __forceinline__ void divmax_block_s(Idx I, const double *ux, const do
     I.dec(t, i, j, k);
     double dv = 0.0;
     if (i > 0 && i < I.mx - 1 && j > 0 && j < I.my - 1 && k > 0 && k < I.mz - 1) {
-      dv = fabs((ux[S * t] - ux[S * (t - 1)] + uy[S * t] - uy[S * (t - sj)] + uz[S * t] - uz[S * (t - sk)]) * aj[t]);
+      dv = fabs((ux[t] - ux[t - 1] + uy[t] - uy[t - sj] + uz[t] - uz[t - sk]) * aj[t]);
       if (nv[t] + nv[t + sk] + nv[t - sk] + nv[t + sj] + nv[t - sj] + nv[t + 1] + nv[t - 1] > 0.1) dv = 0.;
     }
     if (div_beats(dv, t, best, bi)) { best = dv; bi = t; }
@@ -2311,13 +2308,7 @@ __device__ __forceinline__ void divmax_block_s(Idx I, const double *ux, const do
   }
   if (threadIdx.x == 0) { pv[bid] = sv[0]; pi[bid] = (double)si[0]; }
 }
-__device__ __forceinline__ void divmax_block(Idx I, const double *ux, const double *uy, const double *uz,
-                                             const double *aj, const double *nv, long n, double *pv, double *pi,
-                                             int bid, int nb) {
-  divmax_block_s<1>(I, ux, uy, uz, aj, nv, n, pv, pi, bid, nb);
-}
-
-// divmax_block_s<1> as k-marches: block b takes tiles b, b + nb, ... of 64 x
+// divmax_block as k-marches: block b takes tiles b, b + nb, ... of 64 x
 // DV_TY columns by kc planes, and each column's cell takes uz and two
 // nvert planes from the cell below it.  Every point is visited once, and
 // the maximum with its first index does not depend on the visiting order,
@@ -2400,9 +2391,10 @@ int cv_divergence_dev(cv_ctx *c, double *maxdiv, long *idx) {
 // partials live in a file-scope device array, one copy per GPU, that every
 // call on that GPU shares
 // ====================================================================
-#define CV_NOALLOC_PARTS CV_RED_GRID       // (value, index) pairs: 16 KiB per GPU
+#define CV_NOALLOC_BLOCKS 512              // two of 1024 threads per CU
 #define CV_NOALLOC_DEVICES 64
-static __device__ __align__(256) double scratch[2 * CV_NOALLOC_PARTS];
+// (value, index) pairs of the blocks
+static __device__ __align__(256) double scratch[2 * CV_NOALLOC_BLOCKS];
 static double *g_scratch[CV_NOALLOC_DEVICES];   // device address of each GPU's copy
 static std::mutex g_scratch_mu;
 
@@ -2424,33 +2416,87 @@ static int noalloc_scratch(int device, double **out) {
   return CV_OK;
 }
 
-// block partials of Divergence over the DMDA layout (Cmpnts interleaved)
-__global__ static void k_divmax_dmda(Idx I, const double *u, const double *aj, const double *nv, long n,
-                                     double *pv, double *pi) {
-  divmax_block_s<3>(I, u, u + 1, u + 2, aj, nv, n, pv, pi, blockIdx.x, gridDim.x);
+// the better (value, index) of a wave, in every lane
+__device__ inline void div_wave_best(double &v, long &i) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    const double v2 = __shfl_xor(v, o, 64);
+    const long i2 = __shfl_xor(i, o, 64);
+    if (div_beats(v2, i2, v, i)) { v = v2; i = i2; }
+  }
+}
+
+// Divergence over the DMDA layout (Cmpnts interleaved): tiles of 64 x 16
+// interior columns march kc planes; columns past the end repeat the last one
+// (the same value and index), so every load is unconditional, and uz and two
+// nvert planes come from the cell below.  Each XCD takes one contiguous run of
+// tiles (x fastest), its blocks side by side through it, so that the rows two
+// tiles share meet in its L2.  Bound by memory: 40 bytes a point.  512x256x256
+// cells 592 us as a flat pass with 7 nvert and 6 flux reads a point, 314 here
+// (4.4 TB/s; FETCH_SIZE counts 1.17 times the 40 bytes).  32^3 cells stay at
+// their two launches (5.0 and 2.4 us against 4.6 and 4.0).
+// TY: rows of a block, 16, or 4 on grids too small for 512 blocks of 16 rows
+// and 16 planes
+template <int TY>
+__global__ static void __launch_bounds__(64 * TY, 8)
+    k_divmax_dmda(Idx I, const double *__restrict__ u, const double *__restrict__ aj, const double *__restrict__ nv,
+                  int kc, double *pv, double *pi) {
+  __shared__ double sv[TY];
+  __shared__ long si[TY];
+  const int tx = (I.mx - 2 + 63) / 64, ty = (I.my - 2 + TY - 1) / TY, tz = (I.mz - 2 + kc - 1) / kc;
+  const int ntile = tx * ty * tz;
+  // blocks b, b + 8, ... share an XCD: tiles [first, end) in steps of its blocks
+  const int xcd = blockIdx.x % CV_NXCD, lane = blockIdx.x / CV_NXCD, step = ((int)gridDim.x - xcd + CV_NXCD - 1) / CV_NXCD;
+  const int nx = min((int)gridDim.x, CV_NXCD);
+  const int q = ntile / nx, rem = ntile - q * nx;
+  const int first = xcd * q + min(xcd, rem), end = first + q + (xcd < rem ? 1 : 0);
+  const long sj = I.mx, sk = (long)I.mx * I.my;
+  double best = 0.0;     // the ghost point 0 carries 0
+  long bi = 0;
+  for (int tb = first + lane; tb < end; tb += step) {
+    const int bx = tb % tx, by = (tb / tx) % ty, bz = tb / (tx * ty);
+    const int i = min(1 + bx * 64 + (int)threadIdx.x, I.mx - 2), j = min(1 + by * TY + (int)threadIdx.y, I.my - 2);
+    const int k0 = 1 + bz * kc, k1 = min(k0 + kc, I.mz - 1);
+    long t = I.at(i, j, k0);
+    double uzb = u[3 * (t - sk) + 2], nb = nv[t - sk], n0 = nv[t];
+#pragma unroll 2
+    for (int k = k0; k < k1; k++, t += sk) {
+      const double uzt = u[3 * t + 2], nt = nv[t + sk];
+      double dv = fabs((u[3 * t] - u[3 * (t - 1)] + u[3 * t + 1] - u[3 * (t - sj) + 1] + uzt - uzb) * aj[t]);
+      if (n0 + nt + nb + nv[t + sj] + nv[t - sj] + nv[t + 1] + nv[t - 1] > 0.1) dv = 0.;
+      if (div_beats(dv, t, best, bi)) { best = dv; bi = t; }
+      uzb = uzt; nb = n0; n0 = nt;
+    }
+  }
+  div_wave_best(best, bi);
+  if (threadIdx.x == 0) { sv[threadIdx.y] = best; si[threadIdx.y] = bi; }
+  __syncthreads();
+  if (threadIdx.y == 0) {
+    const int w = threadIdx.x & (TY - 1);
+    best = sv[w]; bi = si[w];
+    div_wave_best(best, bi);
+    if (threadIdx.x == 0) { pv[blockIdx.x] = best; pi[blockIdx.x] = (double)bi; }
+  }
 }
 // the largest partial and its first index (the order cv_divergence_dev
-// applies on the host) into out[0], out[1]
-__global__ static void k_divmax_final(const double *pv, const double *pi, int nb, double *out) {
-  __shared__ double sv[BS];
-  __shared__ long si[BS];
-  double best = -1.0;
-  long bi = 0;
-  for (int b = threadIdx.x; b < nb; b += BS) {
-    const long ii = (long)pi[b];
-    if (div_beats(pv[b], ii, best, bi)) { best = pv[b]; bi = ii; }
-  }
-  sv[threadIdx.x] = best;
-  si[threadIdx.x] = bi;
+// applies on the host) into out[0], out[1]; one partial a thread, so that
+// their loads are one round trip
+__global__ static void __launch_bounds__(CV_NOALLOC_BLOCKS)
+    k_divmax_final(const double *pv, const double *pi, int nb, double *out) {
+  __shared__ double sv[CV_NOALLOC_BLOCKS / 64];
+  __shared__ long si[CV_NOALLOC_BLOCKS / 64];
+  const int b = min((int)threadIdx.x, nb - 1);
+  double best = pv[b];
+  long bi = (long)pi[b];
+  div_wave_best(best, bi);
+  if ((threadIdx.x & 63) == 0) { sv[threadIdx.x >> 6] = best; si[threadIdx.x >> 6] = bi; }
   __syncthreads();
-  for (int s = BS / 2; s > 0; s >>= 1) {
-    if (threadIdx.x < s && div_beats(sv[threadIdx.x + s], si[threadIdx.x + s], sv[threadIdx.x], si[threadIdx.x])) {
-      sv[threadIdx.x] = sv[threadIdx.x + s];
-      si[threadIdx.x] = si[threadIdx.x + s];
-    }
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) { out[0] = sv[0]; out[1] = (double)si[0]; }
+  if (threadIdx.x) return;
+  const int nw = blockDim.x / 64;
+  for (int w = 1; w < nw; w++)
+    if (div_beats(sv[w], si[w], best, bi)) { best = sv[w]; bi = si[w]; }
+  out[0] = best;
+  out[1] = (double)bi;
 }
 
 extern "C" int cv_divergence_noalloc(int device, const double *ucont, const double *aj, const double *nvert, int mx,
@@ -2467,13 +2513,20 @@ extern "C" int cv_divergence_noalloc(int device, const double *ucont, const doub
   double *part = nullptr;
   int rc = noalloc_scratch(device, &part);
   if (rc) return rc;
-  const long n = (long)mx * my * mz;
+  // every block writes its own pair, so nothing needs clearing first; a grid
+  // of fewer tiles takes fewer blocks
+  const long cx = (mx - 2 + 63) / 64, c16 = cx * ((my - 2 + 15) / 16);
+  const bool small = c16 * ((mz - 2 + 15) / 16) < CV_NOALLOC_BLOCKS;
+  const long columns = small ? cx * ((my - 2 + 3) / 4) : c16;
+  int kc = cv_march_kchunk(columns, mz - 2, 16, 4 * CV_NOALLOC_BLOCKS);
+  if (small && columns * ((mz - 2 + kc - 1) / kc) < CV_NOALLOC_BLOCKS) kc = 1;   // one plane a block
+  const int nb = (int)std::min<long>(columns * ((mz - 2 + kc - 1) / kc), CV_NOALLOC_BLOCKS);
   hipStream_t s = (hipStream_t)stream;
-  // every block writes its own pair, so nothing needs clearing first
-  hipLaunchKernelGGL(k_divmax_dmda, dim3(CV_NOALLOC_PARTS), dim3(BS), 0, s, Idx{mx, my, mz}, ucont, aj, nvert, n,
-                     part, part + CV_NOALLOC_PARTS);
-  hipLaunchKernelGGL(k_divmax_final, dim3(1), dim3(BS), 0, s, (const double *)part,
-                     (const double *)(part + CV_NOALLOC_PARTS), CV_NOALLOC_PARTS, out);
+  if (small)
+    hipLaunchKernelGGL(k_divmax_dmda<4>, dim3(nb), dim3(64, 4), 0, s, Idx{mx, my, mz}, ucont, aj, nvert, kc, part, part + nb);
+  else
+    hipLaunchKernelGGL(k_divmax_dmda<16>, dim3(nb), dim3(64, 16), 0, s, Idx{mx, my, mz}, ucont, aj, nvert, kc, part, part + nb);
+  hipLaunchKernelGGL(k_divmax_final, dim3(1), dim3((nb + 63) / 64 * 64), 0, s, (const double *)part, (const double *)(part + nb), nb, out);
   CV_CHECK(hipGetLastError());
   return CV_OK;
 }

@@ -194,8 +194,8 @@ int cv_divergence(cv_ctx *ctx, double *maxdiv, long *idx); /* Divergence       m
  * doubles, the maximum |div| and its first storage index (the result of
  * cv_divergence on the same fields, bit for bit).  Runs on `stream` (a
  * hipStream_t; 0 for the null stream) of GPU `device` and returns without
- * waiting.  Its block partials live in a fixed device array of 1024
- * (value, index) pairs (16 KiB) per GPU, held until the process ends and
+ * waiting.  Its block partials live in a fixed device array of 512
+ * (value, index) pairs (8 KiB) per GPU, held until the process ends and
  * shared by every call on that GPU: calls that overlap on one GPU race.
  * Storage of 2^31 points or more, or below 3 per axis, is refused with
  * CV_ERR_ARG. */
