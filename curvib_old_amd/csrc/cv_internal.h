@@ -149,6 +149,8 @@ int cv_prof_drain(cv_ctx *c);
 // helpers implemented in cv_ctx.hip
 int cv_alloc(cv_ctx *c, void **p, size_t bytes);
 void cv_free(cv_ctx *c, void *p);
+// device array to host, after the context's earlier work; complete on return
+int cv_copy_out(cv_ctx *c, void *host, const void *dev, size_t bytes);
 int cv_reduce_sum(cv_ctx *c, const double *const *vecs_a, const double *const *vecs_b, int nvec,
                   long n, double *out_host);
 

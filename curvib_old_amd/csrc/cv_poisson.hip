@@ -2580,9 +2580,8 @@ extern "C" int cv_poisson_apply(cv_ctx *c, int level, const double *x, double *y
   CV_CHECK(hipMemcpyAsync(L.b, x, L.d.n * sizeof(double), hipMemcpyHostToDevice, c->stream));
   stencil<double, 0>(c, level, (const double *)L.b, (const double *)nullptr, L.r);
   CV_CHECK(hipGetLastError());
-  CV_CHECK(hipMemcpyAsync(y, L.r, L.d.n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-  CV_CHECK(hipStreamSynchronize(c->stream));
-  return CV_OK;
+  CV_CHECK(hipGetLastError());
+  return cv_copy_out(c, y, L.r, L.d.n * sizeof(double));
 }
 
 extern "C" int cv_poisson_solve(cv_ctx *c, cv_step_stats *st) {
@@ -2636,9 +2635,8 @@ extern "C" int cv_mg_restrict(cv_ctx *c, int lc, const double *xf, double *xc) {
   hipLaunchKernelGGL(k_restrict<double>, dim3(nblk(C.d.n)), dim3(BS), 0, c->stream, idx_of(C), idx_of(F), C.d.isc,
                      C.d.jsc, C.d.ksc, (const double *)F.nvert, (const float *)F.nwf, (const uint32_t *)C.flags,
                      (const double *)F.r, C.b, C.d.n);
-  CV_CHECK(hipMemcpyAsync(xc, C.b, C.d.n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-  CV_CHECK(hipStreamSynchronize(c->stream));
-  return CV_OK;
+  CV_CHECK(hipGetLastError());
+  return cv_copy_out(c, xc, C.b, C.d.n * sizeof(double));
 }
 
 extern "C" int cv_mg_prolong(cv_ctx *c, int lf, const double *xc, double *xf) {
@@ -2650,9 +2648,8 @@ extern "C" int cv_mg_prolong(cv_ctx *c, int lf, const double *xc, double *xf) {
   hipLaunchKernelGGL(k_prolong<double>, dim3(nblk(F.d.n)), dim3(BS), 0, c->stream, idx_of(F), idx_of(C), C.d.isc,
                      C.d.jsc, C.d.ksc, (const double *)C.nvert, (const uint32_t *)F.flags, (const double *)C.r, F.b, 0,
                      F.d.n);
-  CV_CHECK(hipMemcpyAsync(xf, F.b, F.d.n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-  CV_CHECK(hipStreamSynchronize(c->stream));
-  return CV_OK;
+  CV_CHECK(hipGetLastError());
+  return cv_copy_out(c, xf, F.b, F.d.n * sizeof(double));
 }
 
 extern "C" int cv_nullspace_project(cv_ctx *c, int level, double *x) {
@@ -2663,9 +2660,8 @@ extern "C" int cv_nullspace_project(cv_ctx *c, int level, double *x) {
   CvLevel &L = c->lev[level];
   CV_CHECK(hipMemcpyAsync(L.b, x, L.d.n * sizeof(double), hipMemcpyHostToDevice, c->stream));
   nullspace_dev<double>(c, level, L.b);
-  CV_CHECK(hipMemcpyAsync(x, L.b, L.d.n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-  CV_CHECK(hipStreamSynchronize(c->stream));
-  return CV_OK;
+  CV_CHECK(hipGetLastError());
+  return cv_copy_out(c, x, L.b, L.d.n * sizeof(double));
 }
 
 #include "cv_batch_solve.h"
