@@ -127,14 +127,26 @@ __global__ void __launch_bounds__(TW * 4) kb_stencil(BK_ARGS, int d, int sx, int
                                      A.dinv, (T)0, C.lev[d].kc, bx, by, bz);
 }
 
-// x += omega T^-1 r in place (zg: x = omega T^-1 r)
+// x += omega T^-1 r in place (zg: x = omega T^-1 r); in_r: the cases whose x
+// is in the slot BR instead of BX
 template <class T, int CS, bool HL = false>
-__global__ void __launch_bounds__(1024) kb_yline(BK_ARGS, int d, int sr, T omega, int zg) {
+__global__ void __launch_bounds__(1024) kb_yline(BK_ARGS, int d, int sr, unsigned long long in_r, T omega, int zg) {
   BK_HEAD
   const OpV<T> A = bop<T>(C, d);
-  T *x = bvec<T>(C, d, BX, ctl->jj);
+  T *x = bvec<T>(C, d, (in_r >> c & 1ull) ? BR : BX, ctl->jj);
   yline_reg_tile<T, CS, HL>(A.mx, A.my, A.mz, bvec<T>(C, d, sr, 0), A.ylo, A.yip, A.ycp, x, x,
                             HL ? (T)(omega * A.ysc) : omega, zg, lb, A.yh, A.yc);
+}
+
+// one smoothing sweep from BX to BR, or for the cases not in to_r from BR to BX
+// (cv_sweep.h)
+template <class T, bool HG, int CS, int XC>
+__global__ void __launch_bounds__(1024) kb_sweep(BK_ARGS, int d, unsigned long long to_r, T omega) {
+  BK_HEAD
+  const bool r = to_r >> c & 1ull;
+  const OpV<T> A = bop<T>(C, d);
+  sweep_body<T, HG, CS, XC>(A, bvec<T>(C, d, r ? BX : BR, ctl->jj), bvec<T>(C, d, BB, 0), bvec<T>(C, d, r ? BR : BX, ctl->jj),
+                            HG ? (T)(omega * A.ysc) : omega, lb, (T *)sweep_mem);
 }
 
 // the coarse sweeps and the nullspace rule of the cases whose coarsest level
@@ -159,12 +171,13 @@ __global__ void kb_restrict(BK_ARGS, int d) {
                    bvec<T>(C, d + 1, BB, 0), K.n, (long)lb * BS + threadIdx.x, (long)K.nvb * BS);
 }
 
-// x of depth d += P x of depth d+1 (block table of depth d)
+// x of depth d += P x of depth d+1 (block table of depth d); in_r: the cases
+// whose x of depth d+1 is in the slot BR
 template <class T>
-__global__ void kb_prolong(BK_ARGS, int d) {
+__global__ void kb_prolong(BK_ARGS, int d, unsigned long long in_r) {
   BK_HEAD
   const BLev &F = C.lev[d], &K = C.lev[d + 1];
-  prolong_body<T>(F.I, K.I, K.isc, K.jsc, K.ksc, K.nv, F.fl, (const T *)bvec<T>(C, d + 1, BX, ctl->jj),
+  prolong_body<T>(F.I, K.I, K.isc, K.jsc, K.ksc, K.nv, F.fl, (const T *)bvec<T>(C, d + 1, (in_r >> c & 1ull) ? BR : BX, ctl->jj),
                   bvec<T>(C, d, BX, ctl->jj), 1, F.n, (long)lb * BS + threadIdx.x, (long)F.nvb * BS);
 }
 
@@ -410,6 +423,10 @@ struct cv_batch {
   BDiv *ddiv = nullptr;                       // per-case Divergence operands
   uint32_t *dtab = nullptr;
   BTab st[CV_MAXLEV], vc[CV_MAXLEV], rd[CV_MAXLEV], ln[CV_MAXLEV][3];
+  // one-launch sweeps by rows per thread (8, 16), patches of sweep_cols(swrows) columns; swept: every case of the depth takes them
+  BTab sw[CV_MAXLEV][2], sw_v[CV_MAXLEV][2][2];   // sw_v: as st_v
+  int swrows[CV_MAXLEV][2];
+  bool swept[CV_MAXLEV], swept_co[CV_MAXLEV];   // swept_co: its cases that bottom out, alone
   // the same tables restricted to the cases that go deeper [0] or bottom out [1] at the depth
   BTab st_v[CV_MAXLEV][2], vc_v[CV_MAXLEV][2], rd_v[CV_MAXLEV][2], ln_v[CV_MAXLEV][2][3];
   int lnc[CV_MAXLEV][3];
@@ -493,7 +510,7 @@ static void b_stencil(cv_batch *B, int d, unsigned long long pm, int sx, int sb,
 }
 
 template <class T>
-static void b_line(cv_batch *B, int d, unsigned long long pm, int sr, T om, bool zg) {
+static void b_line(cv_batch *B, int d, unsigned long long pm, int sr, unsigned long long in_r, T om, bool zg) {
   const int var = b_variant(B, d, pm);
   for (int g = 0; g < 3; g++) {
     const BTab &t = var < 0 ? B->ln[d][g] : B->ln_v[d][var][g];
@@ -506,21 +523,40 @@ static void b_line(cv_batch *B, int d, unsigned long long pm, int sr, T om, bool
     if constexpr (sizeof(T) == 4) {
       if (B->opt.precision == CV_MIXED16 && g < 2) {      // FP16 line factors (8 or 16 rows per thread)
         if (g == 0)
-          hipLaunchKernelGGL((kb_yline<T, 8, true>), dim3((unsigned)t.len), blk, 0, B->stream, cs, tb, m, ctl, d, sr, om,
+          hipLaunchKernelGGL((kb_yline<T, 8, true>), dim3((unsigned)t.len), blk, 0, B->stream, cs, tb, m, ctl, d, sr, in_r, om,
                              zg ? 1 : 0);
         else
-          hipLaunchKernelGGL((kb_yline<T, 16, true>), dim3((unsigned)t.len), blk, 0, B->stream, cs, tb, m, ctl, d, sr, om,
+          hipLaunchKernelGGL((kb_yline<T, 16, true>), dim3((unsigned)t.len), blk, 0, B->stream, cs, tb, m, ctl, d, sr, in_r, om,
                              zg ? 1 : 0);
         continue;
       }
     }
     if (g == 0)
-      hipLaunchKernelGGL((kb_yline<T, 8>), dim3((unsigned)t.len), blk, 0, B->stream, cs, tb, m, ctl, d, sr, om, zg ? 1 : 0);
+      hipLaunchKernelGGL((kb_yline<T, 8>), dim3((unsigned)t.len), blk, 0, B->stream, cs, tb, m, ctl, d, sr, in_r, om, zg ? 1 : 0);
     else if (g == 1)
-      hipLaunchKernelGGL((kb_yline<T, 16>), dim3((unsigned)t.len), blk, 0, B->stream, cs, tb, m, ctl, d, sr, om, zg ? 1 : 0);
+      hipLaunchKernelGGL((kb_yline<T, 16>), dim3((unsigned)t.len), blk, 0, B->stream, cs, tb, m, ctl, d, sr, in_r, om, zg ? 1 : 0);
     else
       hipLaunchKernelGGL((kb_yline<T, sizeof(T) == 8 ? 16 : 32>), dim3((unsigned)t.len), blk, 0, B->stream, cs, tb, m,
-                         ctl, d, sr, om, zg ? 1 : 0);
+                         ctl, d, sr, in_r, om, zg ? 1 : 0);
+  }
+}
+
+// one sweep of depth d in one launch: the cases of to_r from BX to BR, the
+// others from BR to BX
+template <class T>
+static void b_sweep(cv_batch *B, int d, unsigned long long pm, unsigned long long to_r, T om) {
+  const bool hg = sizeof(T) == 4 && B->opt.precision == CV_MIXED16;
+  const int var = b_variant(B, d, pm);
+  for (int g = 0; g < 2; g++) {
+    const BTab &t = var < 0 ? B->sw[d][g] : B->sw_v[d][var][g];
+    const unsigned long long m = pm & B->lgm[d][g];
+    if (!BLAUNCH_OK(t, m)) continue;
+    const int cs = g == 0 ? 8 : 16, ny = B->swrows[d][g], xc = sweep_cols(ny);
+    sweep_dispatch<T>(hg, cs, xc, [&](auto h, auto rows, auto cols) {
+      hipLaunchKernelGGL((kb_sweep<T, h(), rows(), cols()>), dim3((unsigned)t.len), dim3(sweep_threads(ny, xc)),
+                         sweep_lds(ny, cs, xc) * sizeof(T), B->stream, (const BCase *)B->dcases, (const uint32_t *)BTAB(t),
+                         m, (const BCtl *)B->dctl, d, to_r, om);
+    });
   }
 }
 
@@ -581,40 +617,59 @@ static bool b_coarse(cv_batch *B, int d, unsigned long long co) {
 }
 
 // the V-cycle of depth d for every case that has it; the cases whose
-// coarsest level is at depth d run the coarse sweeps and the nullspace rule
+// coarsest level is at depth d run the coarse sweeps and the nullspace rule.
+// The cases whose x ends in the slot BR instead of BX: none at depth 0
 template <class T>
-static void b_vcycle(cv_batch *B, int d) {
+static unsigned long long b_vcycle(cv_batch *B, int d) {
   if (B->legs && d == B->legs->d0) {
     b_vcycle_legs<T>(B);
-    return;
+    return 0;
   }
   const cv_solver_opts &o = B->opt;
   const T om = (T)o.omega;
   const unsigned long long in = B->inner[d], co = b_coarse<T>(B, d, B->coarse[d]) ? 0 : B->coarse[d];
   const int npre = o.pre_sweeps, npost = o.post_sweeps, nco = o.coarse_sweeps;
+  const bool one = B->swept[d];   // sweeps as one launch, out of place
   const unsigned long long z = (npre == 0 ? in : 0) | (nco == 0 ? co : 0);
   if (z) b_zero<T>(B, d, z, BX);
   const int nsw = std::max(in ? npre : 0, co ? nco : 0);
   for (int s = 0; s < nsw; s++) {
     const unsigned long long m = (s < npre ? in : 0) | (s < nco ? co : 0);
+    // out of place a case's last sweep writes BX: the one before BR, and so on
+    // the coarse sweeps after the last pre-sweep alone: from BX, so an even number of them
+    const bool tail = !one && B->swept_co[d] && m == co && s >= npre && (s > npre || (nco - npre) % 2 == 0);
+    const unsigned long long to_r =
+        one || tail ? ((npre - 1 - s) % 2 ? in & m : 0) | ((nco - 1 - s) % 2 ? co & m : 0) : 0;
+    if (s > 0 && (one || tail)) {
+      b_sweep<T>(B, d, m, to_r, om);
+      continue;
+    }
     if (s > 0) b_stencil<T, 1>(B, d, m, BX, BB, BR);
-    b_line<T>(B, d, m, s == 0 ? BB : BR, om, s == 0);
+    b_line<T>(B, d, m, s == 0 ? BB : BR, to_r, om, s == 0);
   }
   if (co) b_nullspace<T>(B, d, co, BX);
-  if (!in) return;
+  if (!in) return 0;
   b_stencil<T, 1>(B, d, in, BX, BB, BR);
   hipLaunchKernelGGL(kb_restrict<T>, dim3((unsigned)B->vc[d + 1].len), dim3(BS), 0, B->stream, (const BCase *)B->dcases,
                      (const uint32_t *)BTAB(B->vc[d + 1]), in, (const BCtl *)B->dctl, d);
-  b_vcycle<T>(B, d + 1);
+  const unsigned long long in_r = b_vcycle<T>(B, d + 1);
   {
     const BTab &tp = BPICK(B->vc, B->vc_v, d, in);
     hipLaunchKernelGGL(kb_prolong<T>, dim3((unsigned)tp.len), dim3(BS), 0, B->stream, (const BCase *)B->dcases,
-                       (const uint32_t *)BTAB(tp), in, (const BCtl *)B->dctl, d);
+                       (const uint32_t *)BTAB(tp), in, (const BCtl *)B->dctl, d, in_r);
   }
+  bool at_r = false;
   for (int s = 0; s < npost; s++) {
+    // an odd number of sweeps ends in BR; at depth 0 the first stays in place
+    if (one && !(d == 0 && s == 0 && npost % 2)) {
+      at_r = !at_r;
+      b_sweep<T>(B, d, in, at_r ? in : 0, om);
+      continue;
+    }
     b_stencil<T, 1>(B, d, in, BX, BB, BR);
-    b_line<T>(B, d, in, BR, om, false);
+    b_line<T>(B, d, in, BR, 0, om, false);
   }
+  return at_r ? in : 0;
 }
 
 // Z_jj = M^-1 V_jj (nullspace rule applied) and w = A Z_jj for the cases
@@ -921,9 +976,12 @@ extern "C" int cv_batch_create(cv_ctx *const *cases, int ncases, cv_batch **out)
       for (int b = 0; b < p.second; b++) { tabs.push_back(((uint32_t)p.first << 24) | (uint32_t)b); len++; }
     t.len = (int)len;
   };
+  long swn[CV_MAXLEV] = {}, swc[CV_MAXLEV] = {};   // points of the depth (all, bottoming out): they fill the chip together
   for (int l = 0; l < CV_MAXLEV; l++) {
     B->has[l] = B->inner[l] = B->coarse[l] = 0;
     for (int g = 0; g < 3; g++) { B->lgm[l][g] = 0; B->lnc[l][g] = 1; }
+    for (int g = 0; g < 2; g++) B->swrows[l][g] = 0;
+    B->swept[l] = B->swept_co[l] = true;
   }
   for (int c = 0; c < ncases; c++) {
     cv_ctx *x = cases[c];
@@ -971,6 +1029,13 @@ extern "C" int cv_batch_create(cv_ctx *const *cases, int ncases, cv_batch **out)
       const int g = b.cs == 8 ? 0 : b.cs == 16 ? 1 : 2;
       B->lgm[d][g] |= bit(c);
       B->lnc[d][g] = std::max(B->lnc[d][g], (rows + b.cs - 1) / b.cs);
+      swn[d] += b.n;
+      if (g < 2) B->swrows[d][g] = std::max(B->swrows[d][g], rows);
+      B->swept[d] = swn[d] <= SWEEP_MAX && sweep_fits(L.d) && B->swept[d];
+      if (d == x->nlev - 1) {
+        swc[d] += b.n;
+        B->swept_co[d] = swc[d] <= SWEEP_MAX && sweep_fits(L.d) && B->swept_co[d];
+      }
     }
     CvLevel &F = x->lev[x->nlev - 1];
     if (F.d.xper) B->xper |= bit(c);
@@ -990,7 +1055,7 @@ extern "C" int cv_batch_create(cv_ctx *const *cases, int ncases, cv_batch **out)
   for (int d = 0; d < B->maxlev; d++) {
     // v = -1: every case of the depth; 0: the cases that go deeper; 1: those that bottom out here
     for (int v = -1; v < 2; v++) {
-      std::vector<std::pair<int, int>> st, vc, rd, ln[3];
+      std::vector<std::pair<int, int>> st, vc, rd, ln[3], sw[2];
       const unsigned long long m = v < 0 ? B->has[d] : v == 0 ? B->inner[d] : B->coarse[d];
       for (int c = 0; c < ncases; c++) {
         if (!(m & bit(c))) continue;
@@ -1000,11 +1065,13 @@ extern "C" int cv_batch_create(cv_ctx *const *cases, int ncases, cv_batch **out)
         rd.push_back({c, b.nrd});
         const int g = b.cs == 8 ? 0 : b.cs == 16 ? 1 : 2;
         ln[g].push_back({c, b.lgx});
+        if (v == 1 ? B->swept_co[d] : B->swept[d]) sw[g].push_back({c, sweep_patches(cases[c]->lev[cases[c]->nlev - 1 - d].d, sweep_cols(B->swrows[d][g]))});
       }
       add_tab(v < 0 ? B->st[d] : B->st_v[d][v], st);
       add_tab(v < 0 ? B->vc[d] : B->vc_v[d][v], vc);
       add_tab(v < 0 ? B->rd[d] : B->rd_v[d][v], rd);
       for (int g = 0; g < 3; g++) add_tab(v < 0 ? B->ln[d][g] : B->ln_v[d][v][g], ln[g]);
+      for (int g = 0; g < 2; g++) add_tab(v < 0 ? B->sw[d][g] : B->sw_v[d][v][g], sw[g]);
     }
   }
   for (const uint32_t e : tabs)

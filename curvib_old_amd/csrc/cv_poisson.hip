@@ -1170,6 +1170,7 @@ static int nred(long n) {
 }
 
 #include "cv_coarse.h"
+#include "cv_sweep.h"
 
 // k extent of one stencil block (tunable through CV_STENCIL_KCHUNK)
 static int stencil_kchunk(int mz) {
@@ -1559,6 +1560,24 @@ static void line_solve(cv_ctx *c, int l, const T *r, const T *xi, T *xo, T *tmp,
   }
 }
 
+// one y-line sweep of level l from v.x to v.r in one launch; false where it
+// stays a residual and a line solve (a large level, a kernel timed on it)
+template <class T>
+static bool sweep(cv_ctx *c, MgVecs<T> &v, int l, T om) {
+  CvLevel &L = c->lev[l];
+  if (!sweep_fits(L.d) || (c->prof.kind != CV_PROF_NONE && (c->prof.level == l || l == c->nlev - 1))) return false;
+  const OpV<T> A = opview<T>(c, l);
+  const bool hg = sizeof(T) == 4 && half_coef(c) && L.gh;
+  const int ny = L.d.my - 2, cs = ny <= 16 * 8 ? 8 : 16, xc = sweep_cols(ny);
+  const T omh = om * (hg ? (T)A.ysc : (T)1);
+  sweep_dispatch<T>(hg, cs, xc, [&](auto h, auto rows, auto cols) {
+    hipLaunchKernelGGL((k_sweep<T, h(), rows(), cols()>), dim3((unsigned)sweep_patches(L.d, xc)),
+                       dim3(sweep_threads(ny, xc)), sweep_lds(ny, cs, xc) * sizeof(T), c->stream, A, (const T *)v.x[l],
+                       (const T *)v.b[l], v.r[l], omh);
+  });
+  return true;
+}
+
 // nsweep smoothing sweeps on level l; x in v.x[l] (zero_guess: x is 0), r
 // used as ping-pong.  Red-black: each sweep is two damped half-sweeps, the
 // cells of even (i+j+k) then the odd ones from the updated even ones; out of
@@ -1583,11 +1602,13 @@ static void smooth(cv_ctx *c, MgVecs<T> &v, int l, int nsweep, bool zero_guess) 
       T *tmpv = line_tmp<T>(c, l);
       const bool zg = zero_guess && s == 0;
       const T *rr = (const T *)v.b[l];
-      if (!zg) {
-        stencil<T, 1>(c, l, (const T *)v.x[l], (const T *)v.b[l], tmpv);
-        rr = tmpv;
+      if (zg || !sweep<T>(c, v, l, om)) {
+        if (!zg) {
+          stencil<T, 1>(c, l, (const T *)v.x[l], (const T *)v.b[l], tmpv);
+          rr = tmpv;
+        }
+        line_solve<T>(c, l, rr, (const T *)v.x[l], v.r[l], tmpv, om, zg);
       }
-      line_solve<T>(c, l, rr, (const T *)v.x[l], v.r[l], tmpv, om, zg);
     } else {
       if (zero_guess && s == 0)
         hipLaunchKernelGGL(k_jacobi<T>, dim3(nblk(n)), dim3(BS), 0, c->stream, A, (const T *)v.x[l], (const T *)v.b[l],
