@@ -1223,7 +1223,78 @@ __device__ inline double ptan_v(int mode, double p0, double po, double pf, doubl
   return (a + b - c - d) * (lo || up ? 0.5 : 0.25);
 }
 
-__device__ __forceinline__ void ff1_faces_body(FFArgs A, V3 rhs, int kc, int bx, int by, int bz) {
+// CalcRHS (implicitsolver.c:6449-6741) of one storage point after
+// FormFunction1: Rhs += (-1/dt) du with du = 1.5 u - 2 u_o + 0.5 u_rm1 (BDF2)
+// or u - u_o (first step), then the zero set of the reference's interior and
+// boundary-plane masks (all of them only zero entries, so they commute)
+struct CalcArgs {
+  C3 u, uo, um;
+  double idt;
+  int bdf2, yper;
+};
+__device__ __forceinline__ void calcrhs_point(const G &g, const CalcArgs &K, const double *nv, int i, int j, int k, long t,
+                                              double &rx, double &ry, double &rz) {
+  const int mx = g.mx, my = g.my, mz = g.mz, xper = g.xper, zper = g.zper, yper = K.yper;
+  const C3 u = K.u, uo = K.uo, um = K.um;
+  double d0, d1, d2;
+  if (K.bdf2) {
+    d0 = u.x[t] * 1.5; d0 = d0 + (-2.) * uo.x[t]; d0 = d0 + 0.5 * um.x[t];
+    d1 = u.y[t] * 1.5; d1 = d1 + (-2.) * uo.y[t]; d1 = d1 + 0.5 * um.y[t];
+    d2 = u.z[t] * 1.5; d2 = d2 + (-2.) * uo.z[t]; d2 = d2 + 0.5 * um.z[t];
+  } else {
+    d0 = -1. * uo.x[t] + u.x[t];
+    d1 = -1. * uo.y[t] + u.y[t];
+    d2 = -1. * uo.z[t] + u.z[t];
+  }
+  rx = rx + K.idt * d0; ry = ry + K.idt * d1; rz = rz + K.idt * d2;
+  bool zx = false, zy = false, zz = false;
+  const long sj = g.sj, sk = g.sk;
+  auto nvx = [&]() { return nv[t] + nv[t + 1] > 0.1; };
+  auto nvy = [&]() { return nv[t] + nv[t + sj] > 0.1; };
+  auto nvz = [&]() { return nv[t] + nv[t + sk] > 0.1; };
+  // interior cells (6524-6538)
+  if (i >= 1 && i <= mx - 2 && j >= 1 && j <= my - 2 && k >= 1 && k <= mz - 2) {
+    if (nvx() || (i > mx - 3 && !xper)) zx = true;
+    if (nvy() || (j > my - 3 && !yper)) zy = true;
+    if (nvz() || (k > mz - 3 && !zper)) zz = true;
+  }
+  // i planes (6541-6583): j, k in [0, m-2]
+  if (j <= my - 2 && k <= mz - 2) {
+    if (i == 0) {
+      if (!xper) zx = zy = zz = true;
+      else { if (nvx()) zx = true; if (nvy()) zy = true; if (nvz()) zz = true; }
+    }
+    if (i == mx - 2 && !xper) zx = true;
+    if (i == mx - 1) zx = zy = zz = true;
+  }
+  // j planes (6587-6636): i, k in [0, m-2]
+  if (i <= mx - 2 && k <= mz - 2) {
+    if (j == 0) {
+      if (!yper) zx = zy = zz = true;
+      else { if (nvx()) zx = true; if (nvy()) zy = true; if (nvz()) zz = true; }
+    }
+    if (j == my - 2 && !yper) zy = true;
+    if (j == my - 1) zx = zy = zz = true;
+  }
+  // k planes (6639-6690): i, j in [0, m-2]
+  if (i <= mx - 2 && j <= my - 2) {
+    if (k == 0) {
+      if (!zper) zx = zy = zz = true;
+      else { if (nvx()) zx = true; if (nvy()) zy = true; if (nvz()) zz = true; }
+    }
+    if (k == mz - 2 && !zper) zz = true;
+    if (k == mz - 1) zx = zy = zz = true;
+  }
+  rx = zx ? 0. : rx;
+  ry = zy ? 0. : ry;
+  rz = zz ? 0. : rz;
+}
+
+// CALC: CalcRHS of the cell too, from the Rhs in registers.  9.7 M points: 445 us
+// and 40 for the shell of points around the cells, bound by memory; as a pass
+// over all points CalcRHS read and wrote Rhs again, 293 + 258 us
+template <bool CALC = false>
+__device__ __forceinline__ void ff1_faces_body(FFArgs A, V3 rhs, int kc, int bx, int by, int bz, CalcArgs K = CalcArgs{}) {
   const G &g = A.g;
   // what the cell below (k-1) loaded that this cell reads again: its plane
   // k+1 points (this cell's p, pe, pn, pw, ps), its own p, pe, pn (this
@@ -1286,6 +1357,7 @@ __device__ __forceinline__ void ff1_faces_body(FFArgs A, V3 rhs, int kc, int bx,
     if (nv[t + 1] > 0.1) rx = 0;
     if (nv[t + sj] > 0.1) ry = 0;
     if (nvt > 0.1) rz = 0;
+    if constexpr (CALC) calcrhs_point(g, K, nv, i, j, k, t, rx, ry, rz);
     rhs.x[t] = rx; rhs.y[t] = ry; rhs.z[t] = rz;
     have = true;
     c_pt = pt; c_pet = pet; c_pnt = pnt; c_ptw = ptw; c_pts = pts;
@@ -1294,6 +1366,9 @@ __device__ __forceinline__ void ff1_faces_body(FFArgs A, V3 rhs, int kc, int bx,
   }
 }
 __global__ void __launch_bounds__(BS) k_ff1_faces(FFArgs A, V3 rhs, int kc) { ff1_faces_body(A, rhs, kc, blockIdx.x, blockIdx.y, blockIdx.z); }
+__global__ void __launch_bounds__(BS) k_ff1_calcrhs(FFArgs A, V3 rhs, int kc, CalcArgs K) {
+  ff1_faces_body<true>(A, rhs, kc, blockIdx.x, blockIdx.y, blockIdx.z, K);
+}
 
 
 // the loop state after the main FormFunction1 sweep: the z-face values of
@@ -1409,67 +1484,27 @@ __global__ void k_rk_update(double a, C3 uo, C3 r, V3 u, long n) { rk_update_bod
 
 
 
-// CalcRHS (implicitsolver.c:6449-6741) after FormFunction1: Rhs += (-1/dt)
-// du with du = 1.5 u - 2 u_o + 0.5 u_rm1 (BDF2) or u - u_o (first step),
-// at every storage point, then the zero set of the reference's interior and
-// boundary-plane masks (all of them only zero entries, so they commute)
-__global__ void __launch_bounds__(BS) k_calcrhs(G g, int bdf2, double idt, C3 u, C3 uo, C3 um, const double *nv,
-                                                V3 r, int yper, int kc) {
-  const int mx = g.mx, my = g.my, mz = g.mz, xper = g.xper, zper = g.zper;
-  CV_MARCH(g, kc) {
-    const long t = g.at(i, j, k);
-    double d0, d1, d2;
-    if (bdf2) {
-      d0 = u.x[t] * 1.5; d0 = d0 + (-2.) * uo.x[t]; d0 = d0 + 0.5 * um.x[t];
-      d1 = u.y[t] * 1.5; d1 = d1 + (-2.) * uo.y[t]; d1 = d1 + 0.5 * um.y[t];
-      d2 = u.z[t] * 1.5; d2 = d2 + (-2.) * uo.z[t]; d2 = d2 + 0.5 * um.z[t];
+// CalcRHS of the shell of points around the interior cells (those
+// ff1_faces_body<true> completes), after the periodic faces' Rhs
+__global__ void k_calcrhs_shell(G g, CalcArgs K, const double *nv, V3 r) {
+  const int mx = g.mx, my = g.my, mz = g.mz;
+  const long ni = (long)my * mz, nj = (long)(mx - 2) * mz, nk = (long)(mx - 2) * (my - 2);
+  for (long s = blockIdx.x * (long)blockDim.x + threadIdx.x; s < 2 * (ni + nj + nk); s += (long)gridDim.x * blockDim.x) {
+    int i, j, k;
+    if (s < 2 * ni) {
+      const long q = s % ni;
+      i = s < ni ? 0 : mx - 1; j = (int)(q % my); k = (int)(q / my);
+    } else if (s < 2 * (ni + nj)) {
+      const long q = (s - 2 * ni) % nj;
+      i = 1 + (int)(q % (mx - 2)); j = s - 2 * ni < nj ? 0 : my - 1; k = (int)(q / (mx - 2));
     } else {
-      d0 = -1. * uo.x[t] + u.x[t];
-      d1 = -1. * uo.y[t] + u.y[t];
-      d2 = -1. * uo.z[t] + u.z[t];
+      const long q = (s - 2 * (ni + nj)) % nk;
+      i = 1 + (int)(q % (mx - 2)); j = 1 + (int)(q / (mx - 2)); k = s - 2 * (ni + nj) < nk ? 0 : mz - 1;
     }
-    double rx = r.x[t] + idt * d0, ry = r.y[t] + idt * d1, rz = r.z[t] + idt * d2;
-    bool zx = false, zy = false, zz = false;
-    const long sj = g.sj, sk = g.sk;
-    auto nvx = [&]() { return nv[t] + nv[t + 1] > 0.1; };
-    auto nvy = [&]() { return nv[t] + nv[t + sj] > 0.1; };
-    auto nvz = [&]() { return nv[t] + nv[t + sk] > 0.1; };
-    // interior cells (6524-6538)
-    if (i >= 1 && i <= mx - 2 && j >= 1 && j <= my - 2 && k >= 1 && k <= mz - 2) {
-      if (nvx() || (i > mx - 3 && !xper)) zx = true;
-      if (nvy() || (j > my - 3 && !yper)) zy = true;
-      if (nvz() || (k > mz - 3 && !zper)) zz = true;
-    }
-    // i planes (6541-6583): j, k in [0, m-2]
-    if (j <= my - 2 && k <= mz - 2) {
-      if (i == 0) {
-        if (!xper) zx = zy = zz = true;
-        else { if (nvx()) zx = true; if (nvy()) zy = true; if (nvz()) zz = true; }
-      }
-      if (i == mx - 2 && !xper) zx = true;
-      if (i == mx - 1) zx = zy = zz = true;
-    }
-    // j planes (6587-6636): i, k in [0, m-2]
-    if (i <= mx - 2 && k <= mz - 2) {
-      if (j == 0) {
-        if (!yper) zx = zy = zz = true;
-        else { if (nvx()) zx = true; if (nvy()) zy = true; if (nvz()) zz = true; }
-      }
-      if (j == my - 2 && !yper) zy = true;
-      if (j == my - 1) zx = zy = zz = true;
-    }
-    // k planes (6639-6690): i, j in [0, m-2]
-    if (i <= mx - 2 && j <= my - 2) {
-      if (k == 0) {
-        if (!zper) zx = zy = zz = true;
-        else { if (nvx()) zx = true; if (nvy()) zy = true; if (nvz()) zz = true; }
-      }
-      if (k == mz - 2 && !zper) zz = true;
-      if (k == mz - 1) zx = zy = zz = true;
-    }
-    r.x[t] = zx ? 0. : rx;
-    r.y[t] = zy ? 0. : ry;
-    r.z[t] = zz ? 0. : rz;
+    const long t = g.at(i, j, k);
+    double x = r.x[t], y = r.y[t], z = r.z[t];
+    calcrhs_point(g, K, nv, i, j, k, t, x, y, z);
+    r.x[t] = x; r.y[t] = y; r.z[t] = z;
   }
 }
 
@@ -1809,8 +1844,9 @@ static FFArgs ffargs(cv_ctx *c) {
 }
 
 // FormFunction1: Contra2Cart is skipped (FormBCS already left Ucat of the
-// same Ucont in place; the reference recomputes the identical values)
-int cv_ff1_dev(cv_ctx *c) {
+// same Ucont in place; the reference recomputes the identical values).  K:
+// CalcRHS of the interior cells in the same pass
+static int ff1_dev(cv_ctx *c, const CalcArgs *K) {
   CvLevel &F = c->lev[c->nlev - 1];
   CvMetrics &M = c->m;
   FFArgs A = ffargs(c);
@@ -1838,7 +1874,9 @@ int cv_ff1_dev(cv_ctx *c) {
     // algorithmic bytes per point: p, rct, 9 face coefficients, nvert, Rhs out, the operator word
     CvProfScope ps(c, CV_PROF_FF1, c->nlev - 1, 0, (double)F.d.n * (8.0 * (1 + 3 + 9 + 1 + 3) + 4.0));
     const int kc = march_kc(F.d);
-    hipLaunchKernelGGL(k_ff1_faces, march_grid(F.d.mx, F.d.my, F.d.mz, kc), MARCH_BLOCK, 0, c->stream, A, v3(c->rhs), kc);
+    const dim3 grid = march_grid(F.d.mx, F.d.my, F.d.mz, kc);
+    if (K) hipLaunchKernelGGL(k_ff1_calcrhs, grid, MARCH_BLOCK, 0, c->stream, A, v3(c->rhs), kc, *K);
+    else hipLaunchKernelGGL(k_ff1_faces, grid, MARCH_BLOCK, 0, c->stream, A, v3(c->rhs), kc);
   }
   if (F.d.xper || F.d.zper) {
     long nf = (F.d.xper ? (long)(A.g.my - 2) * (A.g.mz - 2) : 0) + (F.d.zper ? (long)(A.g.my - 2) * (A.g.mx - 2) : 0);
@@ -1846,6 +1884,20 @@ int cv_ff1_dev(cv_ctx *c) {
   }
   CV_CHECK(hipGetLastError());
   return CV_OK;
+}
+int cv_ff1_dev(cv_ctx *c) { return ff1_dev(c, nullptr); }
+
+// faces without an inlet, far-field, slip or outlet: FormBCS changes
+// only ghosts, so a stage's update, its wall flux reset and Contra2Cart
+// run as one k-march and FormBCS makes its ghost pass alone
+static bool rk_ghosts_only(const cv_ctx *c) { return !c->inlet && !c->far && !c->slip && !c->outlet && rk_fused(); }
+static void rk_c2c(cv_ctx *c, double a, double *const base[3], int wx, int wy, int wz) {
+  const CvLevel &F = c->lev[c->nlev - 1];
+  const CvMetrics &M = c->m;
+  const int kc = march_kc(F.d);
+  hipLaunchKernelGGL(k_rk_c2c, march_grid(F.d.mx, F.d.my, F.d.mz, kc), MARCH_BLOCK, 0, c->stream, gview(c), a, c3(base),
+                     c3(c->rhs), v3(c->ucont), wx, wy, wz, c3(M.csi), c3(M.eta), c3(M.zet), (const double *)F.nvert,
+                     v3(c->ucat), kc);
 }
 
 int cv_rk_dev(cv_ctx *c) {
@@ -1859,19 +1911,12 @@ int cv_rk_dev(cv_ctx *c) {
   const int wx = wall_mask(c->bctype[0], c->bctype[1]), wy = wall_mask(c->bctype[2], c->bctype[3]),
             wz = wall_mask(c->bctype[4], c->bctype[5]);
   const long planes = (long)g.my * g.mz + (long)g.mx * g.mz + (long)g.mx * g.my;
-  // faces without an inlet, far-field, slip or outlet: FormBCS changes
-  // only ghosts, so the stage update, the wall flux reset and Contra2Cart
-  // run as one k-march and FormBCS makes its ghost pass alone
-  const bool fused = !c->inlet && !c->far && !c->slip && !c->outlet && rk_fused();
+  const bool fused = rk_ghosts_only(c);
   for (int s = 0; s < 4; s++) {
     if ((rc = cv_ff1_dev(c))) return rc;
     double a = alfa[s] * c->dt * c->st;
     if (fused) {
-      CvMetrics &M = c->m;
-      const int kc = march_kc(F.d);
-      hipLaunchKernelGGL(k_rk_c2c, march_grid(F.d.mx, F.d.my, F.d.mz, kc), MARCH_BLOCK, 0, c->stream, g, a, c3(c->ucont_o),
-                         c3(c->rhs), v3(c->ucont), wx, wy, wz, c3(M.csi), c3(M.eta), c3(M.zet), (const double *)F.nvert,
-                         v3(c->ucat), kc);
+      rk_c2c(c, a, c->ucont_o, wx, wy, wz);
       if ((rc = cv_ghost_update(c, 1, false))) return rc;
       continue;
     }
@@ -1889,12 +1934,12 @@ int cv_rk_dev(cv_ctx *c) {
 int cv_calcrhs_dev(cv_ctx *c) {
   CvLevel &F = c->lev[c->nlev - 1];
   G g = gview(c);
-  int rc = cv_ff1_dev(c);
+  const CalcArgs K{c3(c->ucont), c3(c->ucont_o), c3(c->ucont_rm1), -1. / c->dt, c->steps_done > 0 ? 1 : 0,
+                   c->bctype[2] == 7 ? 1 : 0};
+  int rc = ff1_dev(c, &K);
   if (rc) return rc;
-  const int kc = march_kc(F.d);
-  hipLaunchKernelGGL(k_calcrhs, march_grid(F.d.mx, F.d.my, F.d.mz, kc), MARCH_BLOCK, 0, c->stream, g,
-                     c->steps_done > 0 ? 1 : 0, -1. / c->dt, c3(c->ucont), c3(c->ucont_o), c3(c->ucont_rm1),
-                     (const double *)F.nvert, v3(c->rhs), c->bctype[2] == 7 ? 1 : 0, kc);
+  const long shell = 2 * ((long)g.my * g.mz + (long)(g.mx - 2) * g.mz + (long)(g.mx - 2) * (g.my - 2));
+  hipLaunchKernelGGL(k_calcrhs_shell, dim3(nblk(shell)), dim3(BS), 0, c->stream, g, K, (const double *)F.nvert, v3(c->rhs));
   CV_CHECK(hipGetLastError());
   return CV_OK;
 }
@@ -1923,6 +1968,7 @@ static void copy3(cv_ctx *c, double *const dst[3], double *const src[3]) {
 // iteration when both ||Rhs||_inf and ||dU||_inf grew
 int cv_imprk_dev(cv_ctx *c, cv_step_stats *st) {
   CvLevel &F = c->lev[c->nlev - 1];
+  const bool fused = rk_ghosts_only(c);
   const double alfa[4] = {0.25, 1 / 3., 0.5, 1.};
   int rc = cv_bc_update_dev(c);
   if (rc || (rc = cv_ib_dev(c))) return rc;   // implicitsolver.c:7128-7131
@@ -1939,9 +1985,15 @@ int cv_imprk_dev(cv_ctx *c, cv_step_stats *st) {
     pseudot++;
     for (int s = 0; s < 4; s++) {
       const double a = lambda * alfa[s] * c->dt * c->st;
-      hipLaunchKernelGGL(k_rk_update, dim3(nblk(F.d.n)), dim3(BS), 0, c->stream, a, c3(c->pucont), c3(c->rhs),
-                         v3(c->ucont), F.d.n);
-      if ((rc = cv_bc_update_dev(c))) return rc;
+      if (fused) {   // ImpRK resets no wall fluxes: no wall masks
+        rk_c2c(c, a, c->pucont, 0, 0, 0);
+        rc = cv_ghost_update(c, 1, false);
+      } else {
+        hipLaunchKernelGGL(k_rk_update, dim3(nblk(F.d.n)), dim3(BS), 0, c->stream, a, c3(c->pucont), c3(c->rhs),
+                           v3(c->ucont), F.d.n);
+        rc = cv_bc_update_dev(c);
+      }
+      if (rc) return rc;
       if ((rc = cv_calcrhs_dev(c))) return rc;
     }
     if ((rc = cv_ib_dev(c))) return rc;       // after the stages, implicitsolver.c:7170-7173
