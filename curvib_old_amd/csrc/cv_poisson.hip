@@ -34,6 +34,16 @@ __global__ void cv_k_final_sum(const double *part, int nb, double *out, int nq) 
   if (q >= nq) return;
   final_sum_body(part, nb, out, q);
 }
+// the same, also into pinned host memory, which holds the sums once the stream
+// is synchronised: a copy of 8 to 300 bytes is a launch of its own behind the
+// sums (with the scale factors as arguments instead of a copy back, 10 of 350 us
+// a FGMRES iteration on 32x32x32 cells, 5 of 280 on 64x64x64)
+__global__ void k_final_sum_host(const double *part, int nb, double *out, double *host, int nq) {
+  const int q = blockIdx.x;
+  if (q >= nq) return;
+  final_sum_body(part, nb, out, q);
+  if (threadIdx.x == 0) host[q] = out[q];
+}
 
 namespace {
 
@@ -1061,14 +1071,13 @@ __device__ __forceinline__ void scale_to_body(double *__restrict__ dst, const do
                                      long t0, long step) {
   for (long t = t0; t < n; t += step) dst[t] = src[t] * a;
 }
-__global__ void k_scale_to(double *__restrict__ dst, const double *__restrict__ src, const double *inv, long n) {
-  scale_to_body(dst, src, inv[0], n, blockIdx.x * (long)blockDim.x + threadIdx.x, (long)gridDim.x * blockDim.x);
+__global__ void k_scale_to(double *__restrict__ dst, const double *__restrict__ src, double a, long n) {
+  scale_to_body(dst, src, a, n, blockIdx.x * (long)blockDim.x + threadIdx.x, (long)gridDim.x * blockDim.x);
 }
 // the same, also writing the FP32 copy the mixed V-cycle takes as its
 // right-hand side (the conversion it would otherwise make on entry)
-__global__ void k_scale_to_f32(double *__restrict__ dst, const double *__restrict__ src, const double *inv,
+__global__ void k_scale_to_f32(double *__restrict__ dst, const double *__restrict__ src, double a,
                                float *__restrict__ f32, long n) {
-  const double a = inv[0];
   for (long t = blockIdx.x * (long)blockDim.x + threadIdx.x; t < n; t += (long)gridDim.x * blockDim.x) {
     const double v = src[t] * a;
     dst[t] = v;
@@ -1310,6 +1319,11 @@ static void stencil(cv_ctx *c, int l, const TX *x, const T *b, T *y, T omega = (
 // sum of part[0..nb) -> dsc[slot] (device)
 static void final_sum(cv_ctx *c, const double *part, int nb, double *out, int nq) {
   hipLaunchKernelGGL(cv_k_final_sum, dim3(nq), dim3(BS), 0, c->stream, part, nb, out, nq);
+}
+
+// the same, also to host (pinned: c->red_host)
+static void final_sum_host(cv_ctx *c, const double *part, int nb, double *out, double *host, int nq) {
+  hipLaunchKernelGGL(k_final_sum_host, dim3(nq), dim3(BS), 0, c->stream, part, nb, out, host, nq);
 }
 
 int cv_levels_setup_nvert(cv_ctx *c, const double *nvert_host) {
@@ -1728,17 +1742,17 @@ static int ensure_krylov(cv_ctx *c) {
 }
 
 // one classical Gram-Schmidt pass of w against V_0..V_{nv-1}: h and ||w||^2
-// to dsc[0..nv], then w -= V h and ||w||^2 to dsc[36]
+// to dsc[0..nv] and red_host[0..nv], then w -= V h and ||w||^2 to [36] of both
 static void gram_schmidt_pass(cv_ctx *c, double *w, const double *V, int nv, long n) {
   double *hd = c->dsc;
   {
     CvProfScope ps(c, CV_PROF_ORTH, c->nlev - 1, 0, (double)n * 8.0 * (nv + 1));
     hipLaunchKernelGGL(mdot_tbl[nv - 1], dim3(nred(n)), dim3(BS), 0, c->stream, (const double *)w, V, n, n, c->part);
   }
-  final_sum(c, c->part, nred(n), hd, nv + 1);
+  final_sum_host(c, c->part, nred(n), hd, c->red_host, nv + 1);
   hipLaunchKernelGGL(orth_tbl[nv - 1], dim3(nred(n)), dim3(BS), 0, c->stream, w, V, n, (const double *)hd, n,
                      c->part);
-  final_sum(c, c->part, nred(n), hd + 36, 1);
+  final_sum_host(c, c->part, nred(n), hd + 36, c->red_host + 36, 1);
 }
 
 // FGMRES(m) for A phi = b on the finest level; phi starts at 0
@@ -1757,8 +1771,7 @@ static int fgmres(cv_ctx *c, const double *b, double *x, int *its_out, double *r
   double *hh = c->red_host;         // pinned host
   // ||b||
   hipLaunchKernelGGL(k_sumsq, dim3(nred(n)), dim3(BS), 0, c->stream, b, n, c->part);
-  final_sum(c, c->part, nred(n), hd + 40, 1);
-  CV_CHECK(hipMemcpyAsync(hh, hd + 40, sizeof(double), hipMemcpyDeviceToHost, c->stream));
+  final_sum_host(c, c->part, nred(n), hd + 40, hh, 1);
   CV_CHECK(hipStreamSynchronize(c->stream));
   const double bnorm = std::sqrt(hh[0]);
   *bnorm_out = bnorm;
@@ -1775,14 +1788,11 @@ static int fgmres(cv_ctx *c, const double *b, double *x, int *its_out, double *r
   hipLaunchKernelGGL(k_copy, dim3(nblk(n)), dim3(BS), 0, c->stream, w, b, n);
   double beta = bnorm;
   while (beta > tol && its < c->opt.max_it) {
-    hh[0] = 1.0 / beta;
-    CV_CHECK(hipMemcpyAsync(hd + 48, hh, sizeof(double), hipMemcpyHostToDevice, c->stream));
     if (zf32)
       hipLaunchKernelGGL(k_scale_to_f32, dim3(nblk(n)), dim3(BS), 0, c->stream, V, (const double *)w,
-                         (const double *)(hd + 48), c->lev[top].bf, n);
+                         1.0 / beta, c->lev[top].bf, n);
     else
-      hipLaunchKernelGGL(k_scale_to, dim3(nblk(n)), dim3(BS), 0, c->stream, V, (const double *)w,
-                         (const double *)(hd + 48), n);
+      hipLaunchKernelGGL(k_scale_to, dim3(nblk(n)), dim3(BS), 0, c->stream, V, (const double *)w, 1.0 / beta, n);
     std::fill(g.begin(), g.end(), 0.0);
     g[0] = beta;
     int jj = 0;
@@ -1801,13 +1811,11 @@ static int fgmres(cv_ctx *c, const double *b, double *x, int *its_out, double *r
       const int nv = jj + 1;
       // first CGS pass
       gram_schmidt_pass(c, w, V, nv, n);
-      CV_CHECK(hipMemcpyAsync(hh, hd, 40 * sizeof(double), hipMemcpyDeviceToHost, c->stream));
       CV_CHECK(hipStreamSynchronize(c->stream));
       double wn2 = hh[nv], hn2 = hh[36];
       for (int q = 0; q < nv; q++) H[q * m + jj] = hh[q];
       if (hn2 < 1e-2 * wn2) {      // DGKS: second classical pass when ||w|| fell below 0.1 of itself
         gram_schmidt_pass(c, w, V, nv, n);
-        CV_CHECK(hipMemcpyAsync(hh, hd, 40 * sizeof(double), hipMemcpyDeviceToHost, c->stream));
         CV_CHECK(hipStreamSynchronize(c->stream));
         for (int q = 0; q < nv; q++) H[q * m + jj] += hh[q];
         hn2 = hh[36];
@@ -1816,14 +1824,12 @@ static int fgmres(cv_ctx *c, const double *b, double *x, int *its_out, double *r
       H[(jj + 1) * m + jj] = hn;
       if (!std::isfinite(hn)) return CV_ERR_NONFINITE;
       if (hn > 0) {
-        hh[0] = 1.0 / hn;
-        CV_CHECK(hipMemcpyAsync(hd + 48, hh, sizeof(double), hipMemcpyHostToDevice, c->stream));
         if (zf32)
           hipLaunchKernelGGL(k_scale_to_f32, dim3(nblk(n)), dim3(BS), 0, c->stream, V + (size_t)(jj + 1) * n,
-                             (const double *)w, (const double *)(hd + 48), c->lev[top].bf, n);
+                             (const double *)w, 1.0 / hn, c->lev[top].bf, n);
         else
           hipLaunchKernelGGL(k_scale_to, dim3(nblk(n)), dim3(BS), 0, c->stream, V + (size_t)(jj + 1) * n,
-                             (const double *)w, (const double *)(hd + 48), n);
+                             (const double *)w, 1.0 / hn, n);
       }
       for (int q = 0; q < jj; q++) {
         double a = H[q * m + jj], bb = H[(q + 1) * m + jj];
@@ -1858,8 +1864,7 @@ static int fgmres(cv_ctx *c, const double *b, double *x, int *its_out, double *r
     // true residual
     stencil<double, 1>(c, top, (const double *)x, b, w);
     hipLaunchKernelGGL(k_sumsq, dim3(nred(n)), dim3(BS), 0, c->stream, (const double *)w, n, c->part);
-    final_sum(c, c->part, nred(n), hd + 40, 1);
-    CV_CHECK(hipMemcpyAsync(hh, hd + 40, sizeof(double), hipMemcpyDeviceToHost, c->stream));
+    final_sum_host(c, c->part, nred(n), hd + 40, hh, 1);
     CV_CHECK(hipStreamSynchronize(c->stream));
     beta = std::sqrt(hh[0]);
     rnorm = beta;
@@ -2393,8 +2398,9 @@ int cv_divergence_dev(cv_ctx *c, double *maxdiv, long *idx) {
   hipLaunchKernelGGL(k_divmax_march, dim3(nb), dim3(64, DV_TY), 0, c->stream, idx_of(F), (const double *)c->ucont[0],
                      (const double *)c->ucont[1], (const double *)c->ucont[2], (const double *)F.aj,
                      (const double *)F.nvert, c->part, c->part + nb, kc);
-  std::vector<double> hv(2 * nb);
-  CV_CHECK(hipMemcpyAsync(hv.data(), c->part, 2 * nb * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+  static_assert(2 * CV_RED_GRID <= 2048, "the upper half of red_host holds the partials");
+  double *const hv = c->red_host + 2048;
+  CV_CHECK(hipMemcpyAsync(hv, c->part, 2 * nb * sizeof(double), hipMemcpyDeviceToHost, c->stream));
   CV_CHECK(hipStreamSynchronize(c->stream));
   double best = -1.0;
   long bi = 0;
