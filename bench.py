@@ -466,9 +466,9 @@ def main():
     achieved = (byts / (ms * 1e-3)) / 1e9 if ms > 0 else 0.0
     roof = {
         "bound": "hbm",
-        "kernel": ("k_stencil<float, 1, 4, true, true> (fine-level operator residual r = b - A x of the FP32 "
+        "kernel": ("k_stencil<float, 1, 4, true, 32> (fine-level operator residual r = b - A x of the FP32 "
                    "V-cycle, FP16 face coefficients: 36 B per point)" if args.mixed == "mixed16" else
-                   "k_stencil<float, 1, 4, true> (fine-level operator residual r = b - A x of the FP32 V-cycle: "
+                   "k_stencil<float, 1, 4, false, 32> (fine-level operator residual r = b - A x of the FP32 V-cycle: "
                    "56 B per point)"),
         "launches": launches,
         "avg_us": 1e3 * ms / launches if launches else None,
