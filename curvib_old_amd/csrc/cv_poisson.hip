@@ -1138,6 +1138,11 @@ static inline unsigned nblk(long n) {
   return (unsigned)b;
 }
 
+// FP16 face coefficients and line factors in the FP32 V-cycle
+static bool half_coef(const cv_ctx *c) { return c->opt.precision == CV_MIXED16; }
+
+// the FP16 packs are shown under CV_MIXED16 alone: a context that left it keeps
+// their memory but no longer repacks them
 template <class T>
 static OpV<T> opview(cv_ctx *c, int l);
 template <>
@@ -1156,11 +1161,12 @@ OpV<float> opview<float>(cv_ctx *c, int l) {
   CvLevel &L = c->lev[l];
   OpV<float> A;
   for (int q = 0; q < 9; q++) A.g[q] = L.gf[q];
-  A.hA = L.gh ? (const uint4 *)L.gh : nullptr;
-  A.hB = L.gh ? (const uint2 *)((const char *)L.gh + 16 * L.d.n) : nullptr;
-  A.yh = L.gh ? (const uint32_t *)((const char *)L.gh + 24 * L.d.n) : nullptr;
-  A.yc = L.gh ? (const uint16_t *)((const char *)L.gh + 28 * L.d.n) : nullptr;
-  A.ysc = L.gh ? (float)ldexp(1.0, -L.yexp) : 1.0f;
+  const char *const h = half_coef(c) ? (const char *)L.gh : nullptr;
+  A.hA = h ? (const uint4 *)h : nullptr;
+  A.hB = h ? (const uint2 *)(h + 16 * L.d.n) : nullptr;
+  A.yh = h ? (const uint32_t *)(h + 24 * L.d.n) : nullptr;
+  A.yc = h ? (const uint16_t *)(h + 28 * L.d.n) : nullptr;
+  A.ysc = h ? (float)ldexp(1.0, -L.yexp) : 1.0f;
   A.aj = L.ajf; A.dinv = L.dinvf; A.fl = L.flags;
   A.ylo = L.ylof; A.yip = L.yipf; A.ycp = L.ycpf;
   A.mx = L.d.mx; A.my = L.d.my; A.mz = L.d.mz; A.xper = L.d.xper; A.zper = L.d.zper;
@@ -1260,9 +1266,6 @@ static double stencil_bytes_pt(int mode, bool hg = false) {
   return (double)(mode == 0 ? 12 : mode == 1 ? 13 : 14) * sizeof(T) + 4.0;
 }
 
-// the FP32 V-cycle reads the FP16 face coefficients
-static bool half_coef(const cv_ctx *c) { return c->opt.precision == CV_MIXED16; }
-
 // MODE 0: y = A x; 1: y = b - A x; 2: y = x + omega D^-1 (b - A x), on the
 // cells of one (i+j+k) parity when color is 0 or 1 (the others keep x)
 // tile rows of 32 lanes (31 cells per tile row, two rows per wavefront) by
@@ -1294,7 +1297,7 @@ static void stencil(cv_ctx *c, int l, const TX *x, const T *b, T *y, T omega = (
   dim3 g((unsigned)((L.d.mx + tw - 2) / (tw - 1)), (unsigned)((L.d.my + ty - 1) / ty),
          (unsigned)((L.d.mz + kc - 1) / kc));
   const int remap = stencil_remap(g.x);
-  const bool hg = sizeof(T) == 4 && half_coef(c) && L.gh;
+  const bool hg = A.hA != nullptr;
   CvProfScope ps(c, MODE == 0 ? CV_PROF_APPLY : CV_PROF_RESID, l, sizeof(T) == 4 ? 1 : 0,
                  (double)L.d.n * (stencil_bytes_pt<T>(MODE, hg) - (double)(sizeof(T) - sizeof(TX))));
 #define ST_LAUNCH(TY, HG, TW)                                                                                       \
@@ -1540,7 +1543,7 @@ static void line_solve(cv_ctx *c, int l, const T *r, const T *xi, T *xo, T *tmp,
   const dim3 g((unsigned)(((long)L.d.mx * L.d.mz + 63) / 64));
   const dim3 gs((unsigned)((L.d.mx + 63) / 64), (unsigned)L.d.mz);   // k_yline_solve
   // bytes per point: r, the factors (FP16 packs: 6 bytes, else a, ip, cp), x in and out
-  const bool hl = sizeof(T) == 4 && A.yh && rows <= 16 * 16;
+  const bool hl = A.yh && rows <= 16 * 16;
   CvProfScope ps(c, CV_PROF_LINE, l, sizeof(T) == 4 ? 1 : 0, (double)L.d.n * (hl ? 18.0 : 6.0 * sizeof(T)));
   // FP64 keeps at most 16 rows per thread (32 would spill at 1024 threads)
   const int csmax = sizeof(T) == 8 ? 16 : 32;
@@ -1581,7 +1584,7 @@ static bool sweep(cv_ctx *c, MgVecs<T> &v, int l, T om) {
   CvLevel &L = c->lev[l];
   if (!sweep_fits(L.d) || (c->prof.kind != CV_PROF_NONE && (c->prof.level == l || l == c->nlev - 1))) return false;
   const OpV<T> A = opview<T>(c, l);
-  const bool hg = sizeof(T) == 4 && half_coef(c) && L.gh;
+  const bool hg = A.hA != nullptr;
   const int ny = L.d.my - 2, cs = ny <= 16 * 8 ? 8 : 16, xc = sweep_cols(ny);
   const T omh = om * (hg ? (T)A.ysc : (T)1);
   sweep_dispatch<T>(hg, cs, xc, [&](auto h, auto rows, auto cols) {
@@ -1641,10 +1644,10 @@ template <class T>
 static bool coarse_solve(cv_ctx *c, MgVecs<T> &v) {
   CvLevel &L = c->lev[0];
   const bool line = c->opt.smoother == CV_SMOOTH_YLINE;
-  const bool hg = sizeof(T) == 4 && half_coef(c) && L.gh;
   if (c->opt.smoother == CV_SMOOTH_RB || !coarse_fits<T>(L.d, line)) return false;
   if (c->prof.kind != CV_PROF_NONE && (c->prof.level == 0 || c->nlev == 1)) return false;
   const OpV<T> A = opview<T>(c, 0);
+  const bool hg = A.hA != nullptr;
   const T om = (T)c->opt.omega * (line && hg ? (T)A.ysc : (T)1);
   const CoDims D(L.d.mx, L.d.my, L.d.mz);
   const double inv = c->nfluid[0] > 0 ? 1.0 / c->nfluid[0] : 0.0;
