@@ -442,6 +442,7 @@ static void xf_lane(int device, hipStream_t s, int lane, int lanes, char *host, 
 // on return
 int cv_copy_out(cv_ctx *c, void *host, const void *dev, size_t nbytes) {
   const long bytes = (long)nbytes;
+  CV_CHECK(hipSetDevice(c->device));   // the buffers' events belong to the device current when they are made
   if (bytes >= 4 * XF_CHUNK && bytes % 8 == 0 && (uintptr_t)host % 8 == 0) {
     // memory the runtime knows (pinned, managed, a device pointer) moves directly
     hipPointerAttribute_t at;
