@@ -365,22 +365,26 @@ extern "C" int cv_ctx_destroy(cv_ctx *c) {
 // ---------------------------------------------------------------------
 // The runtime fills pageable memory through its own staging on one thread,
 // which also takes the page faults of the caller's fresh array: 10 GB/s.  Here
-// up to XF_LANES threads each move chunks through a pinned buffer of their own
-// (a kernel writes it over PCIe), so that the faults and copies of one lane
-// overlap the transfers of the others.  p and Ucont of 512x256x256 cells (1.1
-// GB): 103 ms by the runtime, 25 here; of 256x192x192 (310 MB) 30 and 8; of
-// 112x88x88 (29 MB) 1.85 and 1.2.  Chunks through hipMemcpyAsync instead of the
-// kernel cost up to 0.2 ms each (17 ms for the 310 MB); chunks that share a huge
-// page of the destination, 57 ms for the 1.1 GB.
-// One set of buffers (32 MiB) serves the process: a call that finds it in use,
-// or on another GPU, goes through the runtime, and the last context destroyed
-// gives it back.
+// up to XF_LANES threads each move chunks through a part of a pinned block (a
+// kernel writes it over PCIe), so that the faults and copies of one lane overlap
+// the transfers of the others.  p and Ucont of 512x256x256 cells (1.1 GB): 103
+// ms by the runtime, 25 here; of 256x192x192 (310 MB) 30 and 8.  Chunks through
+// hipMemcpyAsync instead of the kernel cost up to 0.2 ms each (17 ms for the 310
+// MB); chunks that share a huge page of the destination, 57 ms for the 1.1 GB.
+// Pinning costs up to 0.1 ms a MiB, and a read may be the only one of its
+// process, so a smaller read takes a smaller block.  The first read, and later
+// ones, in ms, by the runtime | 8 x 4 MiB | 4 x 1 MiB: 16 MiB 1.9, 1.0 | 3.2, 0.5
+// | 1.4, 0.5; 31 MiB 3.4, 2.0 | 4.0, 0.9 | 1.9, 0.9.  Of 783 MiB 77 | 17 | 28.
+// One block serves the process: a call that finds it in use, or on another GPU,
+// goes through the runtime, and the last context destroyed gives it back.
 #define XF_LANES 8
-#define XF_CHUNK (4l << 20)
+#define XF_MIN (16l << 20)       // reads below: the runtime
+#define XF_LARGE (64l << 20)     // XF_LANES chunks of 4 MiB from here on, below 4 of 1 MiB
 static struct {
   std::mutex mu;                 // held for a whole copy
   int device = -1;
-  void *pin[XF_LANES] = {};
+  char *pin = nullptr;
+  long size = 0;                 // bytes of the block
   hipEvent_t ev[XF_LANES] = {};
 } g_xf;
 static std::mutex g_xf_live_mu;
@@ -388,26 +392,35 @@ static long g_xf_live = 0;       // contexts alive
 
 // g_xf.mu held
 static void xf_release() {
-  for (int q = 0; q < XF_LANES; q++) {
-    if (g_xf.ev[q]) (void)hipEventDestroy(g_xf.ev[q]);
-    if (g_xf.pin[q]) (void)hipHostFree(g_xf.pin[q]);
-    g_xf.ev[q] = nullptr;
-    g_xf.pin[q] = nullptr;
+  for (auto &e : g_xf.ev) {
+    if (e) (void)hipEventDestroy(e);
+    e = nullptr;
   }
+  if (g_xf.pin) (void)hipHostFree(g_xf.pin);
+  g_xf.pin = nullptr;
+  g_xf.size = 0;
   g_xf.device = -1;
 }
-// the buffers for `device` (current); false leaves the copy to the runtime
-static bool xf_ready(int device) {
-  if (g_xf.device >= 0) return g_xf.device == device;
-  for (int q = 0; q < XF_LANES; q++)
-    if (hipHostMalloc(&g_xf.pin[q], XF_CHUNK, hipHostMallocDefault) != hipSuccess ||
-        hipEventCreateWithFlags(&g_xf.ev[q], hipEventDisableTiming) != hipSuccess) {
-      (void)hipGetLastError();
-      xf_release();
-      return false;
-    }
+// at least `size` bytes and an event a lane for `device` (current); false
+// leaves the copy to the runtime
+static bool xf_ready(int device, int lanes, long size) {
+  if (g_xf.device >= 0 && g_xf.device != device) return false;
   g_xf.device = device;
-  return true;
+  bool ok = true;
+  if (g_xf.size < size) {
+    if (g_xf.pin) (void)hipHostFree(g_xf.pin);
+    g_xf.pin = nullptr;
+    g_xf.size = 0;
+    ok = hipHostMalloc((void **)&g_xf.pin, (size_t)size, hipHostMallocDefault) == hipSuccess;
+    if (ok) g_xf.size = size;
+  }
+  for (int q = 0; q < lanes && ok; q++)
+    if (!g_xf.ev[q]) ok = hipEventCreateWithFlags(&g_xf.ev[q], hipEventDisableTiming) == hipSuccess;
+  if (!ok) {
+    (void)hipGetLastError();
+    xf_release();
+  }
+  return ok;
 }
 static void xf_context(int delta) {
   std::lock_guard<std::mutex> lk(g_xf_live_mu);
@@ -418,17 +431,17 @@ static void xf_context(int delta) {
   }
 }
 
-// chunks lane, lane + lanes, ... of a copy to the host through the lane's
-// buffer; chunks end at multiples of XF_CHUNK in the host's address space, so
-// no two lanes fault on one huge page
-static void xf_lane(int device, hipStream_t s, int lane, int lanes, char *host, const char *dev, long bytes,
+// chunks lane, lane + lanes, ... of a copy to the host through the lane's part
+// of the block; chunks end at multiples of their size in the host's address
+// space, so lanes share a huge page only where chunks are smaller than one
+static void xf_lane(int device, hipStream_t s, int lane, int lanes, long chunk, char *host, const char *dev, long bytes,
                     hipError_t *err) {
   hipError_t e = hipSetDevice(device);
-  char *const pin = (char *)g_xf.pin[lane];
-  const long skew = (long)((uintptr_t)host % XF_CHUNK);   // chunk q covers [q XF_CHUNK - skew, ...)
-  for (long o = lane * XF_CHUNK - skew; o < bytes && e == hipSuccess; o += lanes * XF_CHUNK) {
+  char *const pin = g_xf.pin + lane * chunk;
+  const long skew = (long)((uintptr_t)host % chunk);   // chunk q covers [q chunk - skew, ...)
+  for (long o = lane * chunk - skew; o < bytes && e == hipSuccess; o += lanes * chunk) {
     const long a = std::max(o, 0l);
-    const size_t m = (size_t)(std::min(o + XF_CHUNK, bytes) - a);
+    const size_t m = (size_t)(std::min(o + chunk, bytes) - a);
     hipLaunchKernelGGL(k_copy, dim3(256), dim3(256), 0, s, (double *)pin, (const double *)(dev + a), (long)(m / 8));
     e = hipGetLastError();
     if (e == hipSuccess) e = hipEventRecord(g_xf.ev[lane], s);
@@ -443,26 +456,27 @@ static void xf_lane(int device, hipStream_t s, int lane, int lanes, char *host, 
 int cv_copy_out(cv_ctx *c, void *host, const void *dev, size_t nbytes) {
   const long bytes = (long)nbytes;
   CV_CHECK(hipSetDevice(c->device));   // the buffers' events belong to the device current when they are made
-  if (bytes >= 4 * XF_CHUNK && bytes % 8 == 0 && (uintptr_t)host % 8 == 0) {
+  if (bytes >= XF_MIN && bytes % 8 == 0 && (uintptr_t)host % 8 == 0) {
     // memory the runtime knows (pinned, managed, a device pointer) moves directly
     hipPointerAttribute_t at;
     const bool pageable = hipPointerGetAttributes(&at, host) != hipSuccess || at.type == hipMemoryTypeUnregistered;
     (void)hipGetLastError();
     std::unique_lock<std::mutex> lk(g_xf.mu, std::defer_lock);
-    if (pageable && lk.try_lock() && xf_ready(c->device)) {
-      const int lanes = (int)std::min<long>(XF_LANES, bytes / XF_CHUNK);
+    const int lanes = bytes >= XF_LARGE ? XF_LANES : 4;
+    const long chunk = (bytes >= XF_LARGE ? 4l : 1l) << 20;
+    if (pageable && lk.try_lock() && xf_ready(c->device, lanes, lanes * chunk)) {
       hipError_t err[XF_LANES] = {};
       std::thread th[XF_LANES];
       int started = 1;
       try {
         for (; started < lanes; started++)
-          th[started] = std::thread(xf_lane, c->device, c->stream, started, lanes, (char *)host, (const char *)dev, bytes,
-                                    &err[started]);
+          th[started] = std::thread(xf_lane, c->device, c->stream, started, lanes, chunk, (char *)host,
+                                    (const char *)dev, bytes, &err[started]);
       } catch (...) {   // no thread to be had: this one moves the rest
       }
-      xf_lane(c->device, c->stream, 0, lanes, (char *)host, (const char *)dev, bytes, &err[0]);
+      xf_lane(c->device, c->stream, 0, lanes, chunk, (char *)host, (const char *)dev, bytes, &err[0]);
       for (int q = started; q < lanes; q++)
-        xf_lane(c->device, c->stream, q, lanes, (char *)host, (const char *)dev, bytes, &err[q]);
+        xf_lane(c->device, c->stream, q, lanes, chunk, (char *)host, (const char *)dev, bytes, &err[q]);
       for (int q = 1; q < started; q++) th[q].join();
       for (int q = 0; q < lanes; q++) CV_CHECK(err[q]);
       return CV_OK;

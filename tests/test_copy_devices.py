@@ -2,7 +2,11 @@
 on stand-ins for the HIP runtime's calls (preloaded, host memory, two devices, a
 current device per thread) that refuse, as the runtime does, an event of one
 device on a stream of another.  Every read returns the bytes that were put,
-whichever device is current."""
+whichever device is current.
+
+What a read pins: pinning takes time a single read does not win back unless the
+block is small beside it, so reads below 64 MiB pin one block of 4 MiB, larger
+ones one of 32 MiB, and further reads none."""
 import os
 import subprocess
 import sys
@@ -25,10 +29,11 @@ static thread_local int cur = 0;
 static thread_local struct { D3 g, b; size_t sh; void *s; } cfg;
 static std::map<const void *, std::string> names;
 static std::mutex mu;
-static long events = 0, pinned = 0, pins = 0;
+static long events = 0, pinned = 0, pins = 0, pin_bytes = 0;
 API long stub_events() { return events; }
 API long stub_pinned() { return pinned; }   // blocks of 64 KiB and more alive
 API long stub_pins() { return pins; }       // and ever made
+API long stub_pin_bytes() { return pin_bytes; }
 API int stub_device() { return cur; }
 API void **__hipRegisterFatBinary(const void *) { static void *m; return &m; }
 API void __hipUnregisterFatBinary(void **) {}
@@ -53,7 +58,7 @@ API int hipHostMalloc(void **p, size_t n, unsigned) {
   *(size_t *)q = n;
   *p = q + 64;
   std::lock_guard<std::mutex> l(mu);
-  if (n >= 1 << 16) { pinned++; pins++; }
+  if (n >= 1 << 16) { pinned++; pins++; pin_bytes += n; }
   return 0;
 }
 API int hipHostFree(void *p) {
@@ -136,6 +141,25 @@ print("reads ok")
 """
 
 
+PINS = r"""
+import ctypes as C, sys
+import numpy as np
+from curvib_old_amd import _lib
+from curvib_old_amd.solver import UserCtx
+
+stub = C.CDLL(sys.argv[1])
+stub.stub_pin_bytes.restype = C.c_long
+u = UserCtx((NODES,) * 3, (7, 7, 1, 1, 7, 7), 1, 100.0, 1e-3)
+z = np.random.default_rng(6).random(u._shape("p", -1))
+u.put("p", z)
+for _ in range(3):
+    assert np.array_equal(u.get("p"), z)
+print("pinned", stub.stub_pins(), stub.stub_pin_bytes(), z.nbytes)
+u.close()
+assert stub.stub_pinned() == 0 and stub.stub_events() == 0
+"""
+
+
 @pytest.fixture(scope="module")
 def stub(tmp_path_factory):
     d = tmp_path_factory.mktemp("hip_stub")
@@ -159,3 +183,13 @@ def test_reads_of_contexts_on_two_devices(stub, mode, nodes):
     driver = DRIVER.replace("NODES", str(nodes)).replace("MIN_BYTES", str(nodes ** 3 * 8))
     r = run_on_stub(stub, driver, mode)
     assert r.returncode == 0 and "reads ok" in r.stdout, (mode, r.stdout[-500:], r.stderr[-1500:])
+
+
+@pytest.mark.skipif(not os.path.exists(_lib.SO_PATH), reason="the library is not built")
+@pytest.mark.parametrize("nodes", [60, 160, 330])    # by the runtime; 33 and 290 MB by threads
+def test_a_read_pins_one_small_block(stub, nodes):
+    r = run_on_stub(stub, PINS.replace("NODES", str(nodes)))
+    assert r.returncode == 0, (r.stdout[-500:], r.stderr[-1500:])
+    blocks, pinned, nbytes = (int(v) for v in r.stdout.split()[-3:])
+    want = 0 if nbytes < 16 << 20 else 4 << 20 if nbytes < 64 << 20 else 32 << 20
+    assert blocks == (want > 0) and pinned == want, (blocks, pinned, nbytes)
