@@ -2456,37 +2456,55 @@ __device__ inline void div_wave_best(double &v, long &i) {
   }
 }
 
-// Divergence over the DMDA layout (Cmpnts interleaved): tiles of 64 x 16
-// interior columns march kc planes; columns past the end repeat the last one
-// (the same value and index), so every load is unconditional, and uz and two
-// nvert planes come from the cell below.  Each XCD takes one contiguous run of
-// tiles (x fastest), its blocks side by side through it, so that the rows two
-// tiles share meet in its L2.  Bound by memory: 40 bytes a point.  512x256x256
-// cells 592 us as a flat pass with 7 nvert and 6 flux reads a point, 314 here
-// (4.4 TB/s; FETCH_SIZE counts 1.17 times the 40 bytes).  32^3 cells stay at
-// their two launches (5.0 and 2.4 us against 4.6 and 4.0).
-// TY: rows of a block, 16, or 4 on grids too small for 512 blocks of 16 rows
-// and 16 planes
-template <int TY>
-__global__ static void __launch_bounds__(64 * TY, 8)
+// n / d for 0 <= n < 2^31 as a product with ceil(2^sh / d), sh = 31 + ceil(log2 d):
+// the factor is below 2^32 and too large by less than 1, so the product is too
+// large by less than 2^31 / 2^sh <= 1 / d, and n / d lies at least 1 / d below
+// the next integer
+struct CvDivisor {
+  unsigned m;
+  int sh;
+  explicit CvDivisor(unsigned d) : sh(31) {
+    while ((1ull << (sh - 31)) < d) sh++;
+    m = (unsigned)(((1ull << sh) + d - 1) / d);
+  }
+  __device__ __forceinline__ unsigned quot(unsigned n) const { return (unsigned)(((unsigned long)n * m) >> sh); }
+};
+
+// Divergence over the DMDA layout (Cmpnts interleaved).  A lane takes one
+// interior column over kc planes: uz and two nvert planes come from the cell
+// below.  The lanes run over the columns of a chunk of planes and on into the
+// next chunk without a gap, whatever the extents; lanes past the end repeat the
+// last column (the same value and index), so every load is unconditional.  Each
+// XCD takes one contiguous run of NT lanes' work after another, its blocks side
+// by side through it, so that the rows and planes two blocks share meet in its
+// L2.  Bound by memory: 40 bytes a point, 4.4 TB/s at 512x256x256 cells.  us a
+// call (two launches), inputs in the caches and not, as a flat pass with 7 nvert
+// and 6 flux reads a point | in tiles of 64 x 16 columns | here:
+//   32^3 cells 8.1, 8.4 | 7.1, 7.3 | 5.9, 6.2
+//   112x88x88 17.8, 17.8 | 20.8, 26.3 | 12.6, 16.2
+//   2x998x998 40.5, 46.4 | 313, 384 | 29.8, 42.4
+//   256x128x128 80, 80 | 57, 75 | 35, 52
+//   512x256x256 587, 587 | 315, 315 | 313, 311
+template <int NT>
+__global__ static void __launch_bounds__(NT, 8)
     k_divmax_dmda(Idx I, const double *__restrict__ u, const double *__restrict__ aj, const double *__restrict__ nv,
-                  int kc, double *pv, double *pi) {
-  __shared__ double sv[TY];
-  __shared__ long si[TY];
-  const int tx = (I.mx - 2 + 63) / 64, ty = (I.my - 2 + TY - 1) / TY, tz = (I.mz - 2 + kc - 1) / kc;
-  const int ntile = tx * ty * tz;
+                  int kc, unsigned items, CvDivisor dx, CvDivisor dy, double *pv, double *pi) {
+  __shared__ double sv[NT / 64];
+  __shared__ long si[NT / 64];
+  const int nx = I.mx - 2, ny = I.my - 2, ntile = (int)((items + NT - 1) / NT);
   // blocks b, b + 8, ... share an XCD: tiles [first, end) in steps of its blocks
   const int xcd = blockIdx.x % CV_NXCD, lane = blockIdx.x / CV_NXCD, step = ((int)gridDim.x - xcd + CV_NXCD - 1) / CV_NXCD;
-  const int nx = min((int)gridDim.x, CV_NXCD);
-  const int q = ntile / nx, rem = ntile - q * nx;
+  const int nxcd = min((int)gridDim.x, CV_NXCD);
+  const int q = ntile / nxcd, rem = ntile - q * nxcd;
   const int first = xcd * q + min(xcd, rem), end = first + q + (xcd < rem ? 1 : 0);
   const long sj = I.mx, sk = (long)I.mx * I.my;
   double best = 0.0;     // the ghost point 0 carries 0
   long bi = 0;
   for (int tb = first + lane; tb < end; tb += step) {
-    const int bx = tb % tx, by = (tb / tx) % ty, bz = tb / (tx * ty);
-    const int i = min(1 + bx * 64 + (int)threadIdx.x, I.mx - 2), j = min(1 + by * TY + (int)threadIdx.y, I.my - 2);
-    const int k0 = 1 + bz * kc, k1 = min(k0 + kc, I.mz - 1);
+    // item: column i of row j of chunk bz
+    const unsigned it = min((unsigned)tb * NT + threadIdx.x, items - 1), r = dx.quot(it), bz = dy.quot(r);
+    const int i = 1 + (int)(it - r * (unsigned)nx), j = 1 + (int)(r - bz * (unsigned)ny);
+    const int k0 = 1 + (int)bz * kc, k1 = min(k0 + kc, I.mz - 1);
     long t = I.at(i, j, k0);
     double uzb = u[3 * (t - sk) + 2], nb = nv[t - sk], n0 = nv[t];
 #pragma unroll 2
@@ -2499,10 +2517,10 @@ __global__ static void __launch_bounds__(64 * TY, 8)
     }
   }
   div_wave_best(best, bi);
-  if (threadIdx.x == 0) { sv[threadIdx.y] = best; si[threadIdx.y] = bi; }
+  if ((threadIdx.x & 63) == 0) { sv[threadIdx.x >> 6] = best; si[threadIdx.x >> 6] = bi; }
   __syncthreads();
-  if (threadIdx.y == 0) {
-    const int w = threadIdx.x & (TY - 1);
+  if (threadIdx.x < 64) {
+    const int w = threadIdx.x & (NT / 64 - 1);
     best = sv[w]; bi = si[w];
     div_wave_best(best, bi);
     if (threadIdx.x == 0) { pv[blockIdx.x] = best; pi[blockIdx.x] = (double)bi; }
@@ -2543,19 +2561,22 @@ extern "C" int cv_divergence_noalloc(int device, const double *ucont, const doub
   double *part = nullptr;
   int rc = noalloc_scratch(device, &part);
   if (rc) return rc;
-  // every block writes its own pair, so nothing needs clearing first; a grid
-  // of fewer tiles takes fewer blocks
-  const long cx = (mx - 2 + 63) / 64, c16 = cx * ((my - 2 + 15) / 16);
-  const bool small = c16 * ((mz - 2 + 15) / 16) < CV_NOALLOC_BLOCKS;
-  const long columns = small ? cx * ((my - 2 + 3) / 4) : c16;
-  int kc = cv_march_kchunk(columns, mz - 2, 16, 4 * CV_NOALLOC_BLOCKS);
-  if (small && columns * ((mz - 2 + kc - 1) / kc) < CV_NOALLOC_BLOCKS) kc = 1;   // one plane a block
-  const int nb = (int)std::min<long>(columns * ((mz - 2 + kc - 1) / kc), CV_NOALLOC_BLOCKS);
+  // One plane a lane and blocks of 256 while the fields fit the 256 MB cache that
+  // serves the planes read again (6 M points: 65x298x298 cells 43 and 65 us, in
+  // the caches and not, against 52 and 69 with 1024 lanes of 8 planes); past it
+  // 16 planes where that leaves four tiles a block, else 8 (200x198x198: 76 and 83
+  // against 85 and 92; 510x248x248: 298 with 8, 306 with 16), in equal chunks.
+  // Every block writes its own pair, so nothing needs clearing first
+  const long cols = (long)(mx - 2) * (my - 2), nz = mz - 2;
+  const bool small = cols * nz <= 6l << 20;
+  const long most = small ? 1 : cols * ((nz + 15) / 16) >= 4l * 1024 * CV_NOALLOC_BLOCKS ? 16 : 8;
+  const long chunks = (nz + most - 1) / most, items = cols * chunks, nt = small ? 256 : 1024;
+  const int kc = (int)((nz + chunks - 1) / chunks);
+  const int nb = (int)std::min<long>((items + nt - 1) / nt, CV_NOALLOC_BLOCKS);
+  const CvDivisor dx((unsigned)(mx - 2)), dy((unsigned)(my - 2));
   hipStream_t s = (hipStream_t)stream;
-  if (small)
-    hipLaunchKernelGGL(k_divmax_dmda<4>, dim3(nb), dim3(64, 4), 0, s, Idx{mx, my, mz}, ucont, aj, nvert, kc, part, part + nb);
-  else
-    hipLaunchKernelGGL(k_divmax_dmda<16>, dim3(nb), dim3(64, 16), 0, s, Idx{mx, my, mz}, ucont, aj, nvert, kc, part, part + nb);
+  hipLaunchKernelGGL((small ? k_divmax_dmda<256> : k_divmax_dmda<1024>), dim3(nb), dim3((unsigned)nt), 0, s,
+                     Idx{mx, my, mz}, ucont, aj, nvert, kc, (unsigned)items, dx, dy, part, part + nb);
   hipLaunchKernelGGL(k_divmax_final, dim3(1), dim3((nb + 63) / 64 * 64), 0, s, (const double *)part, (const double *)(part + nb), nb, out);
   CV_CHECK(hipGetLastError());
   return CV_OK;
