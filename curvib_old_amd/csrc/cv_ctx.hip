@@ -219,6 +219,10 @@ extern "C" int cv_ctx_create(const cv_grid_desc *desc, int device, cv_ctx **out)
   }
   CvDims dims[CV_MAXLEV];
   if (level_dims(desc, dims)) return CV_ERR_ARG;
+  if (dims[desc->mglevels - 1].n > CV_MAX_POINTS) {
+    cv_set_error("cv_ctx_create: %ld storage points, at most %ld", dims[desc->mglevels - 1].n, CV_MAX_POINTS);
+    return CV_ERR_ARG;
+  }
   CV_CHECK(hipSetDevice(device));
   cv_ctx *c = new cv_ctx();
   c->device = device;

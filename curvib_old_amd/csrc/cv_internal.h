@@ -148,6 +148,13 @@ int cv_prof_drain(cv_ctx *c);
 
 // helpers implemented in cv_ctx.hip
 int cv_alloc(cv_ctx *c, void **p, size_t bytes);
+
+// most storage points of a context's finest level: kernels address an FP64 vector
+// by 32-bit byte offsets, the last 16 of which mean outside the grid.  A context
+// takes 800 bytes a point before its Krylov space, so past it no card of less than
+// 430 GB could hold one
+#define CV_MAX_POINTS ((1l << 29) - 2)
+
 void cv_free(cv_ctx *c, void *p);
 // device array to host, after the context's earlier work; complete on return
 int cv_copy_out(cv_ctx *c, void *host, const void *dev, size_t bytes);

@@ -309,6 +309,7 @@ __device__ inline float half_hi(uint32_t w) { return (float)__builtin_bit_cast(_
 // in flight and waits for all, the next plane's prefetch included.
 typedef __amdgpu_buffer_rsrc_t CvBuf;
 #define CV_OOB 0xfffffff0u
+static_assert(CV_MAX_POINTS * 8 <= CV_OOB, "the last FP64 value of the largest level lies below CV_OOB");
 __device__ __forceinline__ CvBuf cv_buf(const void *p, unsigned long bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), 0, (int)(bytes < CV_OOB ? bytes : CV_OOB), 0x00020000);
 }
@@ -715,9 +716,8 @@ __device__ __forceinline__ void yline_reg_tile(int mx, int my, int mz, const T *
   const unsigned q0 = (unsigned)lg * 64u + (unsigned)ti;
   const bool act = q0 < (unsigned)mx * (unsigned)mz;
   const unsigned k = act ? q0 / (unsigned)mx : 0u, i = act ? q0 - k * (unsigned)mx : 0u;
-  // the line's first storage index; a context needs over 256 bytes a point,
-  // so storage stays below 2^29 points on this card and 32-bit byte offsets
-  // of the lanes from a wavefront-uniform row pointer suffice
+  // the line's first storage index: storage holds CV_MAX_POINTS at most, so 32-bit
+  // byte offsets of the lanes from a wavefront-uniform row pointer suffice
   const unsigned base = i + (unsigned)(mx * my) * k;
   const int j0 = 1 + tc * CS;
   const int nrow = max(0, min(CS, my - 1 - j0));

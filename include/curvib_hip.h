@@ -120,6 +120,7 @@ enum {
 };
 
 /* ---- life cycle: MG_Initial (init.c:296-1060) / MG_Finalize (init.c:1063) ---- */
+/* storage of more than 2^29 - 2 points (mx my mz) is refused with CV_ERR_ARG */
 int  cv_ctx_create(const cv_grid_desc *desc, int device, cv_ctx **out);
 int  cv_ctx_destroy(cv_ctx *ctx);
 int  cv_set_solver(cv_ctx *ctx, const cv_solver_opts *opts);
