@@ -578,11 +578,14 @@ extern "C" int cv_put_field(cv_ctx *c, int f, int level, const double *in) {
 // ---------------------------------------------------------------------
 #define CV_PROF_POOL 256
 
+bool cv_prof_on(const cv_ctx *c, int kind, int level, int prec) {
+  const CvProf &P = c->prof;
+  return P.kind == kind && (P.level < 0 ? c->nlev - 1 : P.level) == level && (P.prec < 0 || P.prec == prec);
+}
+
 CvProfScope::CvProfScope(cv_ctx *c_, int kind, int level, int prec, double bytes) : c(c_), on(false) {
   CvProf &P = c->prof;
-  if (P.kind == CV_PROF_NONE || P.kind != kind) return;
-  const int lev = P.level < 0 ? c->nlev - 1 : P.level;
-  if (lev != level || (P.prec >= 0 && P.prec != prec)) return;
+  if (!cv_prof_on(c, kind, level, prec)) return;
   if (P.pending == CV_PROF_POOL && cv_prof_drain(c) != CV_OK) return;
   if (hipEventRecord(P.ev[2 * P.pending], c->stream) != hipSuccess) return;
   on = true;
@@ -611,7 +614,7 @@ int cv_prof_drain(cv_ctx *c) {
 }
 
 extern "C" int cv_prof_select(cv_ctx *c, int kernel, int level, int precision) {
-  if (!c || kernel < CV_PROF_NONE || kernel > CV_PROF_ORTH || level >= c->nlev) return CV_ERR_ARG;
+  if (!c || kernel < CV_PROF_NONE || kernel > CV_PROF_COARSE || level >= c->nlev) return CV_ERR_ARG;
   CV_CHECK(hipSetDevice(c->device));
   int rc = cv_prof_drain(c);
   if (rc) return rc;

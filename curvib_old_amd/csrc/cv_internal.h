@@ -144,6 +144,8 @@ struct CvProfScope {
   CvProfScope(cv_ctx *c, int kind, int level, int prec, double bytes);
   ~CvProfScope();
 };
+// whether the selection is `kind` on that level and precision
+bool cv_prof_on(const cv_ctx *c, int kind, int level, int prec);
 int cv_prof_drain(cv_ctx *c);
 
 // helpers implemented in cv_ctx.hip

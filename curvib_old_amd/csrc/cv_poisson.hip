@@ -1577,16 +1577,27 @@ static void line_solve(cv_ctx *c, int l, const T *r, const T *xi, T *xo, T *tmp,
   }
 }
 
+// whether the residual or the line solve of level l is timed: kernels that hold
+// them step aside
+template <class T>
+static bool launches_timed(const cv_ctx *c, int l) {
+  const int prec = sizeof(T) == 4 ? 1 : 0;
+  return cv_prof_on(c, CV_PROF_RESID, l, prec) || cv_prof_on(c, CV_PROF_LINE, l, prec);
+}
+
 // one y-line sweep of level l from v.x to v.r in one launch; false where it
-// stays a residual and a line solve (a large level, a kernel timed on it)
+// stays a residual and a line solve (a large level, one of the two timed on it)
 template <class T>
 static bool sweep(cv_ctx *c, MgVecs<T> &v, int l, T om) {
   CvLevel &L = c->lev[l];
-  if (!sweep_fits(L.d) || (c->prof.kind != CV_PROF_NONE && (c->prof.level == l || l == c->nlev - 1))) return false;
+  if (!sweep_fits(L.d) || launches_timed<T>(c, l)) return false;
   const OpV<T> A = opview<T>(c, l);
   const bool hg = A.hA != nullptr;
   const int ny = L.d.my - 2, cs = ny <= 16 * 8 ? 8 : 16, xc = sweep_cols(ny);
   const T omh = om * (hg ? (T)A.ysc : (T)1);
+  // bytes per point: the residual's without its result, the line factors, x out
+  CvProfScope ps(c, CV_PROF_SWEEP, l, sizeof(T) == 4 ? 1 : 0,
+                 (double)L.d.n * (stencil_bytes_pt<T>(1, hg) + (hg ? 6.0 : 3.0 * sizeof(T))));
   sweep_dispatch<T>(hg, cs, xc, [&](auto h, auto rows, auto cols) {
     hipLaunchKernelGGL((k_sweep<T, h(), rows(), cols()>), dim3((unsigned)sweep_patches(L.d, xc)),
                        dim3(sweep_threads(ny, xc)), sweep_lds(ny, cs, xc) * sizeof(T), c->stream, A, (const T *)v.x[l],
@@ -1638,20 +1649,23 @@ static void smooth(cv_ctx *c, MgVecs<T> &v, int l, int nsweep, bool zero_guess) 
 }
 
 // the coarse sweeps and the nullspace rule of level 0 in one work-group;
-// false where they stay launches (a large level, the red-black smoother, a
-// kernel timed on that level)
+// false where they stay launches (a large level, the red-black smoother, one of
+// the launches timed on that level)
 template <class T>
 static bool coarse_solve(cv_ctx *c, MgVecs<T> &v) {
   CvLevel &L = c->lev[0];
   const bool line = c->opt.smoother == CV_SMOOTH_YLINE;
   if (c->opt.smoother == CV_SMOOTH_RB || !coarse_fits<T>(L.d, line)) return false;
-  if (c->prof.kind != CV_PROF_NONE && (c->prof.level == 0 || c->nlev == 1)) return false;
+  if (launches_timed<T>(c, 0)) return false;
   const OpV<T> A = opview<T>(c, 0);
   const bool hg = A.hA != nullptr;
   const T om = (T)c->opt.omega * (line && hg ? (T)A.ysc : (T)1);
   const CoDims D(L.d.mx, L.d.my, L.d.mz);
   const double inv = c->nfluid[0] > 0 ? 1.0 / c->nfluid[0] : 0.0;
   const int rows = coarse_rows(L.d, line);
+  // bytes per point: the operator, b, the line factors or the diagonal, x out
+  CvProfScope ps(c, CV_PROF_COARSE, 0, sizeof(T) == 4 ? 1 : 0,
+                 (double)L.d.n * (stencil_bytes_pt<T>(0, hg) + (!line ? 1.0 * sizeof(T) : hg ? 6.0 : 3.0 * sizeof(T))));
   coarse_dispatch<T>(hg, rows, D.faces(), [&](auto hgc, auto cs, auto fpt) {
     hipLaunchKernelGGL((k_coarse<T, hgc(), cs(), fpt()>), dim3(1), dim3(COARSE_NT), D.lds(rows) * sizeof(T), c->stream, A,
                        (const T *)v.b[0], v.x[0], om, c->opt.coarse_sweeps, inv, nred(L.d.n));

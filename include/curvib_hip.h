@@ -297,7 +297,9 @@ int cv_batch_destroy(cv_batch *b);
  * finest; precision -1 = either, 0 = FP64, 1 = FP32.  cv_prof_read returns
  * the launch count, their summed device time in ms and the summed
  * algorithmic bytes (compulsory HBM traffic of the launch's inputs and
- * outputs); reset clears the counters. */
+ * outputs); reset clears the counters.  Where a level runs SWEEP or COARSE,
+ * timing RESID or LINE on it runs their launches instead, with the same
+ * results; every other choice leaves the kernels that run as they are. */
 #define CV_PROF_NONE   0
 #define CV_PROF_RESID  1   /* 19-point operator residual r = b - A x       */
 #define CV_PROF_APPLY  2   /* 19-point operator apply y = A x (Krylov)     */
@@ -305,6 +307,8 @@ int cv_batch_destroy(cv_batch *b);
 #define CV_PROF_RCT    4   /* momentum face-flux pass (Visc - Conv, Rc -> rct) */
 #define CV_PROF_FF1    5   /* momentum face RHS (rct, p -> Rhs)            */
 #define CV_PROF_ORTH   6   /* Gram-Schmidt dot products                    */
+#define CV_PROF_SWEEP  7   /* smoothing sweep of a small level in one launch */
+#define CV_PROF_COARSE 8   /* coarsest level in one work-group             */
 int cv_prof_select(cv_ctx *ctx, int kernel, int level, int precision);
 int cv_prof_read(cv_ctx *ctx, long *launches, double *total_ms, double *bytes, int reset);
 
