@@ -1865,8 +1865,10 @@ static int ff1_dev(cv_ctx *c, const CalcArgs *K) {
     hipLaunchKernelGGL(k_rct_periodic, dim3(nblk((long)A.g.my * A.g.mz + (long)A.g.mx * A.g.my)), dim3(BS), 0, c->stream,
                        A.g, v3(c->rct));
   {
-    // algorithmic bytes per point: p, rct, 9 face coefficients, nvert, Rhs out, the operator word
-    CvProfScope ps(c, CV_PROF_FF1, c->nlev - 1, 0, (double)F.d.n * (8.0 * (1 + 3 + 9 + 1 + 3) + 4.0));
+    // algorithmic bytes per point: p, rct, 9 face coefficients, nvert, Rhs out, the operator word; with CalcRHS
+    // Ucont of this and the last step, under BDF2 of the one before too
+    CvProfScope ps(c, CV_PROF_FF1, c->nlev - 1, 0,
+                   (double)F.d.n * (8.0 * (1 + 3 + 9 + 1 + 3 + (!K ? 0 : K->bdf2 ? 9 : 6)) + 4.0));
     const int kc = march_kc(F.d);
     const dim3 grid = march_grid(F.d.mx, F.d.my, F.d.mz, kc);
     if (K) hipLaunchKernelGGL(k_ff1_calcrhs, grid, MARCH_BLOCK, 0, c->stream, A, v3(c->rhs), kc, *K);

@@ -2,7 +2,9 @@
 level in one work-group are timed as such, and neither that nor timing a kernel
 they do not hold changes what runs.  The counts follow from the cycle: per FGMRES
 iteration one V-cycle, whose first pre-sweep starts from zero and is a line solve
-alone.  Tolerance: exact equality."""
+alone.  The face RHS counts the values CalcRHS reads beside its own: in ImpRK Ucont of
+this and the last step, from the second step on of the one before too.  Tolerance:
+exact equality."""
 import numpy as np
 import pytest
 
@@ -38,5 +40,25 @@ def test_small_levels_kernels_are_timed(precision, cells, levels):
             i, r, p, got = solve(kernel, level)
             assert i == its and r == rnorm and np.array_equal(p, phi), (precision, kernel, level)
             assert got == n if n is not None else got > 0, (precision, kernel, level, got, n)
+    finally:
+        u.close()
+
+
+def test_face_rhs_counts_calcrhs_bytes():
+    case = cases.ChannelCase(cells=(16, 24, 8), amp=0.05, re=300.0, seed=8, dt=2e-4)
+    u, _ = from_case(case, mglevels=1)
+    try:
+        u.set_solver(smoother="yline", rtol=1e-6)
+        u.prof_select("ff1")
+        u.Flow_Solver()
+        n, _, nbytes = u.prof_read(reset=True)
+        pts = np.prod(case.storage)
+        assert n == 4 and nbytes == n * pts * (17 * 8 + 4)
+        u.put("ucont", u.get("ucont"))      # a first step again
+        u.set_momentum(scheme="imprk")
+        for values in (17 + 6, 17 + 9):
+            u.Flow_Solver()
+            n, _, nbytes = u.prof_read(reset=True)
+            assert n > 4 and nbytes == n * pts * (values * 8 + 4), (n, nbytes / n / pts, values)
     finally:
         u.close()
