@@ -48,6 +48,11 @@ ILU(0) Richardson smoothing, one block per thread, RK momentum) timed for
 one fractional step of the same workload at 256x128x128 cells on every host
 thread, scaled by cell count; ``cpu_baseline_1core`` the same on one thread
 at 128x64x64 cells.  Both run before any GPU work.
+
+The result line holds a few thousand characters whatever the number of steps:
+iteration counts as their range, accuracy as its worst step, the serving legs as
+their throughputs and latencies.  ``--detail FILE`` writes every step's and every
+leg's record.
 """
 from __future__ import annotations
 
@@ -331,6 +336,49 @@ def run_serving(serve_reqs, arrivals, ens_reqs, nsteps, ens_steps, mixed="mixed1
     return out
 
 
+def sig(v, digits=5):
+    """v with floats to `digits` significant digits, throughout dicts and lists."""
+    if isinstance(v, dict):
+        return {k: sig(x, digits) for k, x in v.items()}
+    if isinstance(v, (list, tuple)):
+        return [sig(x, digits) for x in v]
+    return float(f"{v:.{digits}g}") if isinstance(v, float) else v
+
+
+def result_line(rec):
+    """The result line of a full record: the same keys, what grows with the steps
+    or the cases in short."""
+    def leg(d):
+        if d is None:
+            return None
+        d = dict(d)
+        if "its" in d:
+            d["its"] = [min(d["its"]), max(d["its"])]
+        rows = d.pop("accuracy", None)
+        if rows:
+            d["p_rel_l2_max"] = max(r["p_rel_l2"] for r in rows)
+        return d
+
+    out = dict(rec)
+    for k in ("fp64", "mixed", "mixed_fp32", "shard_share_8way"):
+        out[k] = leg(rec[k])
+    pc = leg(rec["mixed_fp32_4level_rb"])
+    out["mixed_fp32_4level_rb"] = pc and {k: pc[k] for k in ("mg_levels", "smoother", "steps_per_s", "ms_per_step", "its",
+                                                             "over_fp64", "p_rel_l2_max") if k in pc}
+    rows = rec["accuracy"]
+    out["accuracy"] = rows and {
+        "steps": len(rows), **{k: max(r[k] for r in rows) for k in ("p_rel_l2", "fp64_rel_res", "mixed_rel_res",
+                                                                    "fp64_maxdiv", "mixed_maxdiv")},
+        "its_apart": max(abs(r["fp64_its"] - r["mixed_its"]) for r in rows)}
+    out["serving"] = rec["serving"] and {k: {"cell_updates_per_s": r["cell_updates_per_s"], "makespan_s": r["makespan_s"],
+                                             **({"failed": r["failed"]} if "failed" in r else {})}
+                                         for k, r in rec["serving"].items()}
+    out["step_roofline"] = {k: {"bytes_per_step": r["bytes_per_step"], "achieved": r["achieved"], "frac": r["frac"]}
+                            for k, r in rec["step_roofline"].items()}
+    exact = {k: rec[k] for k in ("value", "ms_per_step")}
+    return json.dumps({**sig(out), **exact})
+
+
 def main():
     ap = argparse.ArgumentParser(description=__doc__.split("\n")[0])
     ap.add_argument("--gpus", type=int, default=1)
@@ -369,6 +417,7 @@ def main():
     ap.add_argument("--ensemble-steps", type=int, default=5)
     ap.add_argument("--ensemble-batch-steps", type=int, default=100,
                     help="timed steps of the batched ensemble (its p99 needs about 100 samples)")
+    ap.add_argument("--detail", default=None, metavar="FILE", help="also write the full record there (JSON)")
     ap.add_argument("--build-workers", type=int, default=min(16, os.cpu_count() or 1))
     args = ap.parse_args()
     SOLVER.update(restart=args.restart, pre_sweeps=args.pre, post_sweeps=args.post, coarse_sweeps=args.coarse,
@@ -540,7 +589,10 @@ def main():
         "gpu_mixed_over_cpu": (sps_mx / cpu["value"]) if cpu else None,
         "gpu_mixed_over_cpu_1core": (sps_mx / cpu1["value"]) if cpu1 else None,
     }
-    print(json.dumps(out), flush=True)
+    if args.detail:
+        with open(args.detail, "w") as f:
+            json.dump(out, f)
+    print(result_line(out), flush=True)
 
 
 if __name__ == "__main__":
