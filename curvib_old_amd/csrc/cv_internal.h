@@ -167,7 +167,8 @@ int cv_reduce_sum(cv_ctx *c, const double *const *vecs_a, const double *const *v
 // fewer while that leaves less than `blocks` blocks for the chip's 256 CUs.
 // A march re-reads a plane where it starts, so long ones move less, but a
 // short grid needs the blocks more.  Momentum of a step with chunks of 16
-// everywhere, and by this rule: 32^3 cells 0.96 and 0.33 ms, 64^3 1.25 and
+// everywhere and the edge averages in twelve rounds, and by this rule with two
+// (0.09 ms less at 32^3 cells): 32^3 cells 0.96 and 0.33 ms, 64^3 1.25 and
 // 0.59, 128x96x96 1.60 and 1.31, 256x192x192 7.83 and 7.69; aiming at 1024
 // blocks instead of 4096 costs the last two 0.1 ms, 4096 face-flux blocks (of
 // 512 threads) instead of 512 cost 128x96x96 0.07 ms.  The chunk never changes

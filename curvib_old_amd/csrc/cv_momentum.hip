@@ -1650,8 +1650,8 @@ int cv_ghost_update(cv_ctx *c, int formbcs, bool cart) {
     if (bxper || bzper)
       hipLaunchKernelGGL(k_periodic_planes, dim3(nblk((long)g.my * g.mz + (long)g.mx * g.my)), dim3(BS), 0, c->stream, g,
                          v3(c->ucat), p, nv);
-    // one block runs the twelve ordered sub-sweeps; 1024 threads cover an
-    // edge line of up to 1024 points in one pass per sub-sweep
+    // one block, as the corners wait for the edges: 1024 threads take the twelve
+    // edges' points 1024 at a time, then the eight corners
     hipLaunchKernelGGL(k_edge_average, dim3(1), dim3(1024), 0, c->stream, g, v3(c->ucat), p);
     if (bxper)
       hipLaunchKernelGGL(k_periodic_full, dim3(nblk(2L * g.mz + 2L * (g.my - 2))), dim3(BS), 0, c->stream, g, 0, formbcs ? 1 : 0,

@@ -722,7 +722,10 @@ __device__ __forceinline__ void yline_reg_tile(int mx, int my, int mz, const T *
   const int j0 = 1 + tc * CS;
   const int nrow = max(0, min(CS, my - 1 - j0));
   // offset of row q of the chunk; rows past the line read row my-1 and are
-  // replaced by the identity, so no load waits behind a branch
+  // replaced by the identity, so no load waits behind a branch.  Where xi is xo
+  // such a load, and any of a lane past the last line (it reads line 0), may meet
+  // its owner's store: what it returns is dropped by `in` and `act`.  A thread's
+  // own rows are stored by it alone, after its loads
   auto row = [&](int q) -> long { return (long)mx * min(j0 + q, my - 1); };
   const long top = (long)mx * (my - 1);
   T av[CS], yv[CS], xv[CS];
@@ -2644,7 +2647,6 @@ extern "C" int cv_poisson_apply(cv_ctx *c, int level, const double *x, double *y
   CvLevel &L = c->lev[level];
   CV_CHECK(hipMemcpyAsync(L.b, x, L.d.n * sizeof(double), hipMemcpyHostToDevice, c->stream));
   stencil<double, 0>(c, level, (const double *)L.b, (const double *)nullptr, L.r);
-  CV_CHECK(hipGetLastError());
   CV_CHECK(hipGetLastError());
   return cv_copy_out(c, y, L.r, L.d.n * sizeof(double));
 }
